@@ -279,6 +279,11 @@ typedef struct mtc_tile_desc {
 
 int mtc_check_tile_desc(const mtc_tile_desc* d);
 
+/* mtc_dequant over the tile stream, with the same result: W_out (K x N fp32, row-major, original
+ * channel order, 16-byte aligned) = W_hat. Writes whole row pieces also where columns are permuted
+ * (gathered-column cells are in Y's order), which the panel stream's units cannot. */
+int mtc_tile_dequant(const mtc_tile_desc* d, float* W_out, void* hip_stream);
+
 /* Bytes of prefill workspace for M rows of X of dtype x_dtype (256-byte aligned
  * workspace; contents need no initialisation): M*K*2 (rounded up to 256) when X may
  * be staged as bf16 first (fp32 X, or a row permutation to gather; fp32 X without a

@@ -17,7 +17,7 @@ ERROR_NAMES = {
 }
 
 EXPORTED = ("mtc_abi_version", "mtc_last_error", "mtc_check_desc", "mtc_dequant", "mtc_gemv_lds_bytes",
-            "mtc_gemv_workspace_bytes", "mtc_gemv_f32", "mtc_gemv_f32_group", "mtc_check_tile_desc", "mtc_gemm_workspace_bytes",
+            "mtc_gemv_workspace_bytes", "mtc_gemv_f32", "mtc_gemv_f32_group", "mtc_check_tile_desc", "mtc_tile_dequant", "mtc_gemm_workspace_bytes",
             "mtc_gemm_bf16", "mtc_gemm_group_workspace_bytes", "mtc_gemm_bf16_group", "mtc_gemv_batch_plan",
             "mtc_gemv_f32_batch", "mtc_gemv_noalloc_scratch_bytes", "mtc_gemv_f32_noalloc", "mtc_gemm_batch_plan",
             "mtc_gemm_bf16_batch", "mtc_gemm_f32_workspace_bytes", "mtc_gemm_f32",
@@ -133,6 +133,8 @@ def declare(lib: ctypes.CDLL) -> None:
     lib.mtc_gemm_bf16_batch.argtypes = [vp, vp, vp]
     lib.mtc_check_tile_desc.restype = i32
     lib.mtc_check_tile_desc.argtypes = [TileDescP]
+    lib.mtc_tile_dequant.restype = i32
+    lib.mtc_tile_dequant.argtypes = [TileDescP, vp, vp]
     lib.mtc_gemm_workspace_bytes.restype = sz
     lib.mtc_gemm_workspace_bytes.argtypes = [TileDescP, i32, i32]
     lib.mtc_gemm_bf16.restype = i32

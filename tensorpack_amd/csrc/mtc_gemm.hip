@@ -18,6 +18,7 @@
 //   k_tile_dequant_bf16 : prefill whose 256-row tiles fill the chip many times over decodes
 //                 W_hat once into bf16 and multiplies it with a plain hipBLASLt GEMM instead
 //                 (the tile kernel would decode each weight step once per row tile).
+//   k_tile_dequant_rows : W_hat in fp32 rows (mtc_tile_dequant).
 //
 // Reference behaviour: mtc/kernels/gemm.py:124-210 (block loop: skip P0 blocks,
 // unpack, scale, multiply-accumulate) with W_hat as in mtc/core/quadtree.py:157-171.
@@ -755,9 +756,24 @@ __global__ __launch_bounds__(kStageThreads) void k_stage_x_f32(const float* __re
 // the descriptors of the step after it are in flight. (Stores straight from registers, one cell
 // per thread, ran 54 us against 40 us for one step per block at 8192 x 8192 in bf16: a step's
 // cells are sorted by class first, so their lines split.)
-template <int kCF, bool F32>
+enum { kOutWtBf16, kOutWtF32, kOutRows };   // what tile_dequant_block writes (kOutRows: see below)
+
+// kOutRows: W_hat itself, fp32, row-major in the original channel order (W: K rows of ldw floats).
+// Bound by HBM: 4096 x 4096 QT-P @ 4.25 reads 27 MB and writes 67 MB in 17.9 us, 5.2 TB/s (a 1 GiB
+// copy reaches 5.0; the panel stream's k_dequant and its zero fill took 280 us, its 4-byte stores
+// scattered through col_perm). The
+// LDS tile is then [64 rows][256 columns] and leaves as 1 KiB pieces of rows. Its 16-byte segment
+// `seg` (4 columns) of row `row` sits at seg ^ 2 (row / 8): the lanes of a store take the 8 row
+// blocks of neighbouring column groups (the order of a class's cells), whose segments differ
+// in the bits this leaves alone, so 16 lanes land in 16 segments.
+__device__ __forceinline__ uint32_t swz_rows(int row, int seg) {
+  return (uint32_t)(row * (kTN * 4) + ((seg ^ ((row >> 3) << 1)) << 4));
+}
+
+template <int kCF, int OUT>
 __device__ __forceinline__ void tile_dequant_block(const mtc_tile_desc& d, void* __restrict__ Wt, int64_t ldw,
                                                    int spb) {
+  constexpr bool F32 = OUT != kOutWtBf16;
   __shared__ __attribute__((aligned(16))) unsigned char bs[kTN * kTK * (F32 ? 4 : 2)];
   constexpr int CW = cell_words(kCF);
   const int t = threadIdx.x, ct = blockIdx.x;
@@ -814,7 +830,23 @@ __device__ __forceinline__ void tile_dequant_block(const mtc_tile_desc& d, void*
       }
       const uint32_t pos = (w[h][0] >> 16) & (kCells - 1);   // (column group, row block) of the cell
       const int col = (int)(pos >> 3) * 4, seg = (int)(pos & 7u);
-      if constexpr (F32) {
+      if constexpr (OUT == kOutRows) {
+        // code times scale, as the panel stream's dequantizer computes it (one rounded product: exact for
+        // bf16 scales; no negative zeros in a quadtree W_hat, whose levels are summed into +0.0)
+        const float one[4] = {1.0f, 1.0f, 1.0f, 1.0f};
+        float o[4][8];
+        decode_cell_f32<kCF == kCellCols>((w[h][0] >> 14) & 3u, q[h], one, one, o);
+#pragma unroll
+        for (int r = 0; r < 8; ++r) {
+          f32x4_t v;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            v[j] = o[j][r] * (r < 4 ? st[j] : sb[j]);
+            if constexpr (kCF != kCellFp32) v[j] += 0.0f;
+          }
+          *reinterpret_cast<f32x4_t*>(bs + swz_rows(8 * seg + r, col >> 2)) = v;
+        }
+      } else if constexpr (F32) {
         float o[4][8];
         decode_cell_f32<kCF == kCellCols>((w[h][0] >> 14) & 3u, q[h], st, sb, o);
 #pragma unroll
@@ -833,6 +865,24 @@ __device__ __forceinline__ void tile_dequant_block(const mtc_tile_desc& d, void*
   // 16-byte pieces of the tile's rows: 8 per row in bf16, 16 in fp32
   constexpr int SH = F32 ? 4 : 3, EPP = F32 ? 4 : 8;   // log2 pieces per row, elements per piece
   auto write_out = [&](int ks) __attribute__((always_inline)) {
+    if constexpr (OUT == kOutRows) {
+      const int n = ct * kTN + 4 * (t & 63);               // N % 32 == 0: a segment is wholly inside or outside N
+      if (n >= d.N) return;
+#pragma unroll
+      for (int i = 0; i < kTK / 4; ++i) {
+        const int row = 4 * i + (t >> 6), k = ks * kTK + row;   // one row per wave
+        if (k >= d.K) return;
+        const f32x4_t v = *reinterpret_cast<const f32x4_t*>(bs + swz_rows(row, t & 63));
+        float* const w = reinterpret_cast<float*>(Wt) + (int64_t)(d.row_perm ? d.row_perm[k] : k) * ldw;
+        if (d.col_perm) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) w[d.col_perm[n + j]] = v[j];
+        } else {
+          __builtin_nontemporal_store(v, reinterpret_cast<f32x4_t*>(w + n));
+        }
+      }
+      return;
+    }
 #pragma unroll
     for (int i = 0; i < (kTN << SH) / 256; ++i) {
       const int piece = t + 256 * i, row = piece >> SH, seg = piece & ((1 << SH) - 1);
@@ -868,13 +918,18 @@ __device__ __forceinline__ void tile_dequant_block(const mtc_tile_desc& d, void*
 template <int kCF>
 __global__ __launch_bounds__(256) void k_tile_dequant_bf16(const mtc_tile_desc d, __bf16* __restrict__ Wt,
                                                           int64_t ldw, int spb) {
-  tile_dequant_block<kCF, false>(d, Wt, ldw, spb);
+  tile_dequant_block<kCF, kOutWtBf16>(d, Wt, ldw, spb);
 }
 
 template <int kCF>
 __global__ __launch_bounds__(256) void k_tile_dequant_f32(const mtc_tile_desc d, float* __restrict__ Wt,
                                                          int64_t ldw, int spb) {
-  tile_dequant_block<kCF, true>(d, Wt, ldw, spb);
+  tile_dequant_block<kCF, kOutWtF32>(d, Wt, ldw, spb);
+}
+
+template <int kCF>
+__global__ __launch_bounds__(256) void k_tile_dequant_rows(const mtc_tile_desc d, float* __restrict__ W, int spb) {
+  tile_dequant_block<kCF, kOutRows>(d, W, d.N, spb);
 }
 
 // Up to kMaxGroup matrices that read the same X, in one launch of each kernel: member i owns
@@ -2006,6 +2061,29 @@ MTC_API int mtc_gemm_f32(const mtc_tile_desc* d, const float* X, int64_t ldx, fl
   hipLaunchKernelGGL(k_splitk_reduce<MTC_DTYPE_F32>, dim3((unsigned)reduce_blocks(M, d->N, d->col_perm != nullptr)),
                      dim3(kReduceThreads), 0, st, part, p.splits, M, d->N, d->col_perm, Y, ldy);
   return check_launch("k_splitk_reduce");
+}
+
+MTC_API int mtc_tile_dequant(const mtc_tile_desc* d, float* W_out, void* hip_stream) {
+  int rc = check_tile_desc(d);
+  if (rc) return rc;
+  if (!W_out) return fail(MTC_E_NULL, "W_out is NULL");
+  if (reinterpret_cast<uintptr_t>(W_out) & 15) return fail(MTC_E_SHAPE, "W_out must be 16-byte aligned");
+  // one K-step per block: two blocks fit a CU by LDS (a 64 KiB tile each)
+  const int64_t n_steps = (int64_t)d->n_col_tiles * d->n_ksteps;
+  const int spb = (int)std::min<int64_t>(8, std::max<int64_t>(1, n_steps / (2 * kFillCUs)));
+  const dim3 grid((unsigned)d->n_col_tiles, (unsigned)((d->n_ksteps + spb - 1) / spb));
+  hipStream_t st = reinterpret_cast<hipStream_t>(hip_stream);
+  switch (cell_format(d)) {
+    case kCellFp32:
+      hipLaunchKernelGGL(k_tile_dequant_rows<kCellFp32>, grid, dim3(256), 0, st, *d, W_out, spb);
+      break;
+    case kCellCols:
+      hipLaunchKernelGGL(k_tile_dequant_rows<kCellCols>, grid, dim3(256), 0, st, *d, W_out, spb);
+      break;
+    default:
+      hipLaunchKernelGGL(k_tile_dequant_rows<kCellBf16>, grid, dim3(256), 0, st, *d, W_out, spb);
+  }
+  return check_launch("k_tile_dequant_rows");
 }
 
 MTC_API size_t mtc_gemm_workspace_bytes(const mtc_tile_desc* d, int M, int x_dtype) {

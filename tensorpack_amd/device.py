@@ -323,6 +323,15 @@ class DeviceTiles:
             return None, 0
         return prefill_workspace(self.device, need), need
 
+    def dequant(self):
+        """W_hat as a (K, N) fp32 tensor in the original channel order (mtc_tile_dequant): the
+        bits DeviceStream.dequant gives."""
+        torch = _torch()
+        out = torch.empty((self.K, self.N), dtype=torch.float32, device=self.device)
+        rc = self.lib.mtc_tile_dequant(ctypes.byref(self.desc), out.data_ptr(), current_stream_handle(self.device))
+        _abi.check(self.lib, "mtc_tile_dequant", rc)
+        return out
+
     def gemm_bf16(self, X, out=None, out_dtype=None):
         torch = _torch()
         _need(X.dim() == 2 and X.stride(1) == 1 and X.dtype in (torch.float32, torch.bfloat16) and X.shape[1] == self.K
