@@ -320,15 +320,17 @@ int mtc_gemm_bf16(const mtc_tile_desc* d, const void* X, int x_dtype, int64_t ld
 int mtc_set_prefill_decode_once(int enable);
 
 /* fp32 matrix-core path over the tile stream: Y (M x N fp32, leading dim ldy) = X (M x K
- * fp32, leading dim ldx) * W_hat with the exact fp32 W_hat and fp32 products and sums
- * (v_mfma_f32_16x16x4f32), in 16-row tiles with K split over blocks until the chip is full;
- * within the fp32 tolerance of the reference's float32 block loop (mtc/kernels/gemm.py:124-210,
- * the same operation as mtc_gemv_f32, for callers at 5..16 rows and beyond). X read in place
+ * fp32, leading dim ldx) * W_hat with the exact fp32 W_hat, fp32 X and fp32 sums: both are cut into
+ * bf16 planes whose products are exact in fp32 (v_mfma_f32_32x32x16_bf16 over plane pairs; pairs below
+ * 2^-24 of the product are left out), in tiles of 32, 64 or 128 rows with K split over blocks until the
+ * chip is full; within the fp32 tolerance of the reference's float32 block loop
+ * (mtc/kernels/gemm.py:124-210, the same operation as mtc_gemv_f32, for callers at 5..16 rows and
+ * beyond). Values that are not finite give what a plain fp32 loop gives. X read in place
  * must have 16-byte aligned rows (ldx % 4 == 0); a stream with a row permutation gathers X
  * into the workspace first. Workspace (mtc_gemm_f32_workspace_bytes, 256-byte aligned, no
  * initialisation): the gathered X (M*K*4) and the split-K partials.
- * Decode-once path: a call with M >= 256, M * K * N >= 2^32 and no col_perm decodes the exact
- * W_hat once into fp32 in the workspace (N*64*ceil(K/64)*4 bytes, then the gathered X) and runs
+ * Decode-once path: a call with M >= 256, K <= 1024, M * K * N >= 2^32 and no col_perm decodes the
+ * exact W_hat once into fp32 in the workspace (N*64*ceil(K/64)*4 bytes, then the gathered X) and runs
  * hipBLASLt's fp32 GEMM on it (fp32 products and sums); deterministic, one algorithm per shape;
  * without hipBLASLt, or with the path switched off (mtc_set_prefill_decode_once), the tile
  * kernel runs. */

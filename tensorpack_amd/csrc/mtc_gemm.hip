@@ -19,6 +19,7 @@
 //                 W_hat once into bf16 and multiplies it with a plain hipBLASLt GEMM instead
 //                 (the tile kernel would decode each weight step once per row tile).
 //   k_tile_dequant_rows : W_hat in fp32 rows (mtc_tile_dequant).
+//   k_gemm_f32  : fp32 results (mtc_gemm_f32), from bf16 planes of X and W_hat (mtc_gemm_short.h).
 //
 // Reference behaviour: mtc/kernels/gemm.py:124-210 (block loop: skip P0 blocks,
 // unpack, scale, multiply-accumulate) with W_hat as in mtc/core/quadtree.py:157-171.
@@ -100,13 +101,10 @@ __device__ __forceinline__ uint32_t swz(int row, int seg) {
   return (uint32_t)(row * 128 + ((seg ^ (row & 7) ^ ((row >> 3) & 1)) << 4));
 }
 
-// fp32 tiles of the matrix-core fp32 path: [rows][64] floats, 256 bytes (all 64 banks) per row,
-// 16-byte segment `seg` (0..15) of row `row` stored at segment seg ^ f(row), f(row) = (row & 15)
-// ^ bit 2 of row: the 16 rows that one MFMA operand read takes at one segment land in 16
-// different segments (f is a bijection on 0..15), and so do the producers' stores of one column
-// of two neighbouring cells (rows n and n + 4, whose f differ in bit 0, at the 8 even or the 8
-// odd segments).
-constexpr int kTileBytesF32 = kTN * kTK * 4;             // one fp32 B tile (64 KiB)
+// fp32 tiles of the decode-once path: [rows][64] floats, 256 bytes (all 64 banks) per row, 16-byte
+// segment `seg` (0..15) of row `row` stored at segment seg ^ f(row), f(row) = (row & 15) ^ bit 2 of
+// row, so that the stores of one column of two neighbouring cells (rows n and n + 4, whose f differ in
+// bit 0, at the 8 even or the 8 odd segments) land in different segments.
 __device__ __forceinline__ uint32_t swz_f32(int row, int seg) {
   return (uint32_t)(row * 256 + ((seg ^ (row & 15) ^ ((row >> 2) & 1)) << 4));
 }
@@ -298,10 +296,9 @@ __device__ __forceinline__ bool tile_of_block(int bx, int n_row_tiles, int n_ct,
 }
 
 // The producer waves of a tile block (pid: 0 .. kProducers-1): load the step's cell descriptors and
-// payload, decode the cells of step k+1 into B buffer (k+1) & 1 at bbase (bf16 [256][64] tiles, or
-// with F32 fp32 [256][64] tiles in swz_f32 order) while the consumers multiply step k, and
-// meet the consumers at one LDS-only barrier per step.
-template <int kCF, bool F32>
+// payload, decode the cells of step k+1 into B buffer (k+1) & 1 at bbase (bf16 [256][64] tiles) while
+// the consumers multiply step k, and meet the consumers at one LDS-only barrier per step.
+template <int kCF>
 __device__ __forceinline__ void tile_producers(const mtc_tile_desc& d, const int ct, const int kb0, const int nks,
                                                unsigned char* bbase, const int pid) {
   constexpr int CW = cell_words(kCF);                     // words loaded per cell
@@ -373,24 +370,13 @@ __device__ __forceinline__ void tile_producers(const mtc_tile_desc& d, const int
     }
     const uint32_t pos = w[0] >> 16;
     const int col = (int)(pos >> 3) * 4, seg = (int)(pos & 7u);
-    if constexpr (F32) {
-      float o[4][8];
-      decode_cell_f32<kCF == kCellCols>((w[0] >> 14) & 3u, q, st, sb, o);
+    u32x4_t o[4];
+    decode_cell<kCF == kCellCols>((w[0] >> 14) & 3u, q, st, sb, o);
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int n = col + j;
-        *reinterpret_cast<f32x4_t*>(bs + swz_f32(n, 2 * seg)) = f32x4_t{o[j][0], o[j][1], o[j][2], o[j][3]};
-        *reinterpret_cast<f32x4_t*>(bs + swz_f32(n, 2 * seg + 1)) = f32x4_t{o[j][4], o[j][5], o[j][6], o[j][7]};
-      }
-    } else {
-      u32x4_t o[4];
-      decode_cell<kCF == kCellCols>((w[0] >> 14) & 3u, q, st, sb, o);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) *reinterpret_cast<u32x4_t*>(bs + swz(col + j, seg)) = o[j];
-    }
+    for (int j = 0; j < 4; ++j) *reinterpret_cast<u32x4_t*>(bs + swz(col + j, seg)) = o[j];
   };
   auto fill = [&](int buf, const uint32_t (&w0)[CW], const uint32_t (&w1)[CW]) {
-    unsigned char* bs = bbase + buf * (F32 ? kTileBytesF32 : kTileBytes);
+    unsigned char* bs = bbase + buf * kTileBytes;
     stage_cell(bs, w0, q0);
     stage_cell(bs, w1, q1);
   };
@@ -604,7 +590,7 @@ __device__ __forceinline__ void gemm_tile_block(const mtc_tile_desc& d, const in
     return;
   }
 
-  tile_producers<kCF, false>(d, ct, kb0, nks, lds + kABufs * kTileBytes, tid - 64 * kConsumerWaves);
+  tile_producers<kCF>(d, ct, kb0, nks, lds + kABufs * kTileBytes, tid - 64 * kConsumerWaves);
 }
 
 // One output tile block of matrix `d`: output tile (rt, ct) of TM rows, K split by; X is bf16,
@@ -619,117 +605,18 @@ __global__ __launch_bounds__(kThreads) void k_gemm_tile(const mtc_tile_desc d, c
   gemm_tile_block<kCF, kYDT, TM, kXF>(d, rt, ct, (int)blockIdx.y, X, ldx, Y, ldy, M, steps_per_split, part);
 }
 
-// ---------------------------------------------------------------------------
-// fp32 matrix-core path over the tile stream (mtc_gemm_f32): Y = X * W_hat with fp32 X and
-// the exact fp32 W_hat, on v_mfma_f32_16x16x4f32 (fp32 products and sums) - the decode-size
-// counterpart of k_gemm_tile for callers that need the fp32 result (M of a few to 16 rows per
-// tile). Block = one 16 x 256 output tile, K in steps of 64, the same warp split as k_gemm_tile:
-// 4 producer waves decode step k+1's cells into an fp32 B tile ([256][64], swz_f32) while 8
-// consumer waves multiply step k; consumer wave w owns output columns 32w .. 32w+31 (two 16 x 16
-// MFMA tiles). Waves 0-3 copy the step's X tile ([16][64] fp32, swz_f32; 4 KiB, one 1 KiB copy
-// each) straight into LDS two steps ahead. MFMA lane l takes A[l % 16][l / 16] and
-// B[l / 16][l % 16] and holds D[4 (l / 16) + r][l % 16] in register r (checked on the GPU); each
-// 16-row group g of a step is 4 MFMAs in which lane quarter q contributes K rows 16g + 4q + s
-// (s = 0..3), so one 16-byte LDS read gives a lane its operand for all four.
-// ---------------------------------------------------------------------------
-constexpr int kFM = 16;                                   // output rows per fp32 tile
-constexpr int kABytesF32 = kFM * kTK * 4;                 // one fp32 X tile (4 KiB)
-constexpr int kLdsBytesF32 = kABufs * kABytesF32 + kBBufs * kTileBytesF32;   // 140 KiB
+#include "mtc_gemm_short.h"
 
-template <int kCF>
-__device__ __forceinline__ void gemm_f32_block(const mtc_tile_desc& d, const int rt, const int ct, const int by,
-                                               const float* __restrict__ X, int64_t ldx, float* __restrict__ Y,
-                                               int64_t ldy, int M, int steps_per_split, float* __restrict__ part) {
-  extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int m0 = rt * kFM, n0 = ct * kTN;
-  const int kb0 = by * steps_per_split;
-  const int nks = min(steps_per_split, d.n_ksteps - kb0);
-  unsigned char* const bbase = lds + kABufs * kABytesF32;
-
-  if (wave < kConsumerWaves) {
-    // X copies: wave w < 4 copies rows 4w .. 4w+3 of each step's tile; lane l fills physical
-    // segment l % 16 of row 4w + l / 16, reading the logical segment swz_f32 maps there.
-    // Rows past M and segments past K read zeros.
-    const bool copies = wave < kFM / 4;
-    const uint32_t lds0 = (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)lds;
-    const u32x4_t x_r = buffer_rsrc(X + (int64_t)m0 * ldx, (uint32_t)(kFM * ldx * 4));
-    const int xrow = 4 * wave + (lane >> 4);
-    const int xseg = (lane & 15) ^ (xrow & 15) ^ ((xrow >> 2) & 1);   // logical segment (swz_f32): K 4 xseg .. +3
-    const uint32_t x_off = copies && m0 + xrow < M ? (uint32_t)(xrow * ldx + 4 * xseg) * 4 : kOutOfRange;
-    auto copy_x = [&](int s) __attribute__((always_inline)) {
-      if (!copies) return;
-      const bool in = x_off != kOutOfRange && (kb0 + s) * kTK + 4 * xseg < d.K;   // K % 8 == 0
-      dma16(x_r, in ? x_off + (uint32_t)((kb0 + s) * kTK) * 4 : kOutOfRange,
-            __builtin_amdgcn_readfirstlane(lds0 + (uint32_t)(s % kABufs) * kABytesF32 + (uint32_t)wave * 1024u));
-    };
-    f32x4_t acc[2] = {f32x4_t{0.0f, 0.0f, 0.0f, 0.0f}, f32x4_t{0.0f, 0.0f, 0.0f, 0.0f}};
-    const int r16 = lane & 15, q = lane >> 4;
-    copy_x(0);
-    if (nks > 1) {
-      copy_x(1);
-      asm volatile("s_waitcnt vmcnt(1)" ::: "memory");    // step 0's copy done (waves without copies: none)
-    } else {
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    }
-    lds_barrier();                                         // step 0 staged
-    for (int ks = 0; ks < nks; ++ks) {
-      const bool ahead = ks + 2 < nks;
-      if (ahead) copy_x(ks + 2);                           // into the buffer step ks-1 used
-      const unsigned char* as = lds + (ks % kABufs) * kABytesF32;
-      const unsigned char* bs = bbase + (ks & 1) * kTileBytesF32;
-      // the step's operands first (12 reads in flight), then its 32 MFMAs
-      f32x4_t a[kTK / 16], b[kTK / 16][2];
-#pragma unroll
-      for (int g = 0; g < kTK / 16; ++g) {
-        a[g] = *reinterpret_cast<const f32x4_t*>(as + swz_f32(r16, 4 * g + q));
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-          b[g][t] = *reinterpret_cast<const f32x4_t*>(bs + swz_f32(32 * wave + 16 * t + r16, 4 * g + q));
-      }
-#pragma unroll
-      for (int g = 0; g < kTK / 16; ++g)
-#pragma unroll
-        for (int s = 0; s < 4; ++s)
-#pragma unroll
-          for (int t = 0; t < 2; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[g][s], b[g][t][s], acc[t], 0, 0, 0);
-      if (ahead) {
-        asm volatile("s_waitcnt vmcnt(1)" ::: "memory");  // step ks+1's copy (issued a step ago) landed
-      } else {
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      }
-      lds_barrier();                                       // buffers of step ks free, step ks+1 staged
-    }
-    // epilogue: register r of lane l is row 4 (l / 16) + r, column l % 16 of each 16 x 16 tile.
-    // Split K writes a plain fp32 partial tile to part[by] (no column permutation).
-    float* const yf = part ? part + (size_t)by * M * d.N : Y;
-    const int64_t ld = part ? (int64_t)d.N : ldy;
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      const int col = n0 + 32 * wave + 16 * t + r16;
-      if (col >= d.N) continue;
-      const int ycol = (d.col_perm && !part) ? d.col_perm[col] : col;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int row = m0 + 4 * q + r;
-        if (row < M) yf[(int64_t)row * ld + ycol] = acc[t][r];
-      }
-    }
-    return;
-  }
-
-  tile_producers<kCF, true>(d, ct, kb0, nks, bbase, tid - 64 * kConsumerWaves);
-}
-
-template <int kCF>
-__global__ __launch_bounds__(kThreads) void k_gemm_f32(const mtc_tile_desc d, const float* __restrict__ X, int64_t ldx,
-                                                       float* __restrict__ Y, int64_t ldy, int M, int n_row_tiles,
-                                                       int tiles_per_xcd, int steps_per_split,
-                                                       float* __restrict__ part) {
+// fp32 results (mtc_gemm_f32): Y = X * W_hat with fp32 X and the exact W_hat.
+template <int kCF, int TM>
+__global__ __launch_bounds__((ShortTile<kXSplit, TM>::threads)) void k_gemm_f32(const mtc_tile_desc d, const float* __restrict__ X,
+                                                            int64_t ldx, float* __restrict__ Y, int64_t ldy, int M,
+                                                            int n_row_tiles, int tiles_per_xcd, int steps_per_split,
+                                                            float* __restrict__ part) {
   int rt, ct;
   if (!tile_of_block((int)blockIdx.x, n_row_tiles, d.n_col_tiles, tiles_per_xcd, d.col_perm && !part, rt, ct)) return;
-  gemm_f32_block<kCF>(d, rt, ct, (int)blockIdx.y, X, ldx, Y, ldy, M, steps_per_split, part);
+  gemm_short_block<kCF, MTC_DTYPE_F32, kXSplit, TM>(d, rt, ct, (int)blockIdx.y, X, ldx, Y, ldy, M, steps_per_split,
+                                                    part);
 }
 
 // Xp[m, k] = X[m, row_perm[k]] in fp32 (four outputs per thread), for the fp32 tile path over a
@@ -1532,15 +1419,18 @@ int decode_once_call(const mtc_tile_desc* d, const void* X, int x_dtype, int64_t
 }
 
 // ---- decode once for fp32 results (mtc_gemm_f32): the exact W_hat in fp32, then hipBLASLt's
-// fp32 GEMM (fp32 products and sums, like the tile path), for calls with at least
-// kDecodeOnceF32MinRows rows, kDecodeOnceF32MinMacs multiply-adds and no output column
-// permutation (an fp32 GEMM of 4096 x 4096 x M took 75 us at M = 256 against 176 us for the fp32
-// tile kernel, and 24 against 52 us at M = 64, where writing the 64 MB W_hat costs 20 us more).
+// fp32 GEMM (fp32 products and sums), for calls with at least kDecodeOnceF32MinRows rows,
+// kDecodeOnceF32MinMacs multiply-adds, no output column permutation and K of at most kDecodeOnceF32MaxK.
+// The tile kernel is the faster one at every size (4096 x 4096 QT @ 4.5, M = 256, 1024, 2048: 53, 165, 284 us
+// against 85, 248, 476; 1024 x 4096, M = 1024: 49 against 76); the path stays where K <= 1024 for callers
+// that read the decoded W_hat from the workspace, as the decode-once tests do.
 constexpr int kDecodeOnceF32MinRows = 256;
+constexpr int kDecodeOnceF32MaxK = 1024;
 constexpr int64_t kDecodeOnceF32MinMacs = (int64_t)1 << 32;
 
 bool decode_once_f32_shape(const mtc_tile_desc* d, int M) {
-  return !d->col_perm && M >= kDecodeOnceF32MinRows && (int64_t)M * d->K * d->N >= kDecodeOnceF32MinMacs;
+  return !d->col_perm && d->K <= kDecodeOnceF32MaxK && M >= kDecodeOnceF32MinRows &&
+         (int64_t)M * d->K * d->N >= kDecodeOnceF32MinMacs;
 }
 
 // Workspace of the fp32 path: Wt (N x ldw fp32), then X gathered through row_perm (M x K fp32).
@@ -1945,18 +1835,43 @@ MTC_API int mtc_gemm_bf16_batch(const void* host_plan, const void* device_plan, 
 MTC_API int mtc_check_tile_desc(const mtc_tile_desc* d) { return check_tile_desc(d); }
 
 // ---- fp32 tile path (k_gemm_f32) ----
-// K splits of an fp32 call: enough (16-row tile, column tile, split) blocks to fill the chip, at
-// least kMinStepsPerSplit K-steps each.
+// Tile height and K split of an fp32 call: the height (32, 64 or 128 rows) and split count (at most
+// enough blocks to fill the chip, at least kMinStepsPerSplit K-steps each) with the least estimated time, as
+// tile_plan estimates it.
 struct F32Plan {
+  int tm;        // output rows per tile block
   int splits;
   int per;       // K-steps per split
 };
-F32Plan f32_plan(const mtc_tile_desc* d, int M) {
-  const int64_t n_tiles = (int64_t)((M + kFM - 1) / kFM) * d->n_col_tiles;
-  int s = n_tiles >= kFillCUs ? 1 : (int)((kFillCUs + n_tiles - 1) / n_tiles);
-  s = std::max(1, std::min(s, d->n_ksteps / kMinStepsPerSplit));
-  const int per = (d->n_ksteps + s - 1) / s;
-  return {(d->n_ksteps + per - 1) / per, per};
+// Time of one K-step of an fp32 block by its row-tile height (one block alone over 128 steps): decode
+// 1.2-1.4 us, then the MFMAs, 0.5 us for 32 rows, 1.1 for 64 and 2.2 (their peak rate) for 128. kF32BlockUs:
+// launch to the first step's data; the partials move faster than the bf16 path's (4096 x 4096, M = 100 with
+// 16 splits of 128 rows 39.1 us, 8 of 64 rows 39.2, 4 of 32 rows 45.3; M = 256 59.8, 62.0, 76.4).
+constexpr double kF32BlockUs = 7.0;
+constexpr double kF32ReduceBytesPerUs = 5.0e6;
+inline double f32_step_us(int tm) { return tm == 128 ? 3.6 : tm == 64 ? 2.4 : 1.75; }
+F32Plan f32_plan(const mtc_tile_desc* d, int M, int64_t ldx = 0) {
+  const double split_bytes = 2.0 * 4.0 * (double)M * d->N;     // one partial, written and read
+  F32Plan best{0, 1, d->n_ksteps};
+  double best_t = 1e300;
+  for (int tm : {32, 64, 128}) {
+    if (tm > 32 && (M <= tm / 2 || ldx >= ((int64_t)1 << 30) / tm)) break;   // 32-bit offsets within a block's X rows
+    const int64_t n_tiles = (int64_t)((M + tm - 1) / tm) * d->n_col_tiles;
+    int max_s = n_tiles >= kFillCUs ? 1 : (int)((kFillCUs + n_tiles - 1) / n_tiles);
+    max_s = std::max(1, std::min(max_s, d->n_ksteps / kMinStepsPerSplit));
+    for (int s = 1; s <= max_s; ++s) {
+      const int per = (d->n_ksteps + s - 1) / s;
+      const int s_eff = (d->n_ksteps + per - 1) / per;
+      const double rounds = std::ceil((double)(n_tiles * s_eff) / kFillCUs);
+      const double t = rounds * (per * f32_step_us(tm) + kF32BlockUs) +
+                       (s_eff > 1 ? s_eff * split_bytes / kF32ReduceBytesPerUs + kReduceLaunchUs : 0.0);
+      if (t < best_t) {
+        best_t = t;
+        best = {tm, s_eff, per};
+      }
+    }
+  }
+  return best;
 }
 // Workspace of an fp32 call: X gathered through row_perm (M*K*4, rounded up to 256), then the
 // split-K partials (splits*M*N*4).
@@ -1967,6 +1882,32 @@ size_t f32_ws_bytes(const mtc_tile_desc* d, int M) {
   const F32Plan p = f32_plan(d, M);
   return f32_stage_bytes(d, M) + (p.splits > 1 ? (size_t)p.splits * M * d->N * 4 : 0);
 }
+
+namespace {
+template <int kCF>
+int launch_f32(const mtc_tile_desc* d, const F32Plan& p, const float* X, int64_t ldx, float* Y, int64_t ldy, int M,
+               float* part, hipStream_t st) {
+  const void* fn = p.tm == 128  ? reinterpret_cast<const void*>(&k_gemm_f32<kCF, 128>)
+                   : p.tm == 64 ? reinterpret_cast<const void*>(&k_gemm_f32<kCF, 64>)
+                                : reinterpret_cast<const void*>(&k_gemm_f32<kCF, 32>);
+  const int lds = p.tm == 128  ? ShortTile<kXSplit, 128>::lds_bytes
+                  : p.tm == 64 ? ShortTile<kXSplit, 64>::lds_bytes
+                               : ShortTile<kXSplit, 32>::lds_bytes;
+  if ((size_t)lds > mtc::host::device_lds_limit())
+    return fail(MTC_E_SHAPE, "fp32 tile kernel needs %d B of LDS per block, device has %zu", lds,
+                mtc::host::device_lds_limit());
+  int nrt = (M + p.tm - 1) / p.tm;
+  const int64_t n_tiles = (int64_t)nrt * d->n_col_tiles;
+  if (n_tiles > (int64_t)1 << 30) return fail(MTC_E_SHAPE, "M=%d gives too many tiles", M);
+  int tpx = (int)((n_tiles + kXcds - 1) / kXcds), spp = p.per;
+  hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  if (e != hipSuccess) return fail(MTC_E_LAUNCH, "hipFuncSetAttribute: %s", hipGetErrorString(e));
+  void* args[] = {const_cast<mtc_tile_desc*>(d), &X, &ldx, &Y, &ldy, &M, &nrt, &tpx, &spp, &part};
+  e = hipLaunchKernel(fn, dim3(tpx * kXcds, p.splits), dim3(ShortTile<kXSplit, 32>::threads), args, lds, st);
+  if (e != hipSuccess) return fail(MTC_E_LAUNCH, "k_gemm_f32 launch: %s", hipGetErrorString(e));
+  return check_launch("k_gemm_f32");
+}
+}  // namespace
 
 MTC_API size_t mtc_gemm_f32_workspace_bytes(const mtc_tile_desc* d, int M) {
   if (check_tile_desc(d) || M <= 0) return 0;
@@ -1983,11 +1924,8 @@ MTC_API int mtc_gemm_f32(const mtc_tile_desc* d, const float* X, int64_t ldx, fl
   if (ldx < d->K || ldy < d->N) return fail(MTC_E_SHAPE, "ldx=%lld < K or ldy=%lld < N", (long long)ldx, (long long)ldy);
   if (!d->row_perm && (ldx % 4 || (reinterpret_cast<uintptr_t>(X) & 15)))
     return fail(MTC_E_SHAPE, "fp32 X read in place needs 16-byte aligned rows (ldx=%lld)", (long long)ldx);
-  if (ldx >= ((int64_t)1 << 31) / (4 * kFM))
+  if (ldx >= (int64_t)1 << 25)
     return fail(MTC_E_SHAPE, "ldx=%lld too large for 32-bit X tile offsets", (long long)ldx);
-  if ((size_t)kLdsBytesF32 > mtc::host::device_lds_limit())
-    return fail(MTC_E_SHAPE, "fp32 tile kernel needs %d B of LDS per block, device has %zu", kLdsBytesF32,
-                mtc::host::device_lds_limit());
   hipStream_t st = reinterpret_cast<hipStream_t>(hip_stream);
   const lt::Plan* once = nullptr;
   if (decode_once_f32_shape(d, M) && g_decode_once.load(std::memory_order_relaxed))
@@ -2041,22 +1979,13 @@ MTC_API int mtc_gemm_f32(const mtc_tile_desc* d, const float* X, int64_t ldx, fl
     xa = xp;
     lda = d->K;
   }
-  const F32Plan p = f32_plan(d, M);
+  const F32Plan p = f32_plan(d, M, lda);   // a longer row only lowers the tile height, and with it the splits
   float* part = p.splits > 1 ? reinterpret_cast<float*>(reinterpret_cast<char*>(workspace) + stage) : nullptr;
-  const int n_row_tiles = (M + kFM - 1) / kFM;
-  const int64_t n_tiles = (int64_t)n_row_tiles * d->n_col_tiles;
-  if (n_tiles > (int64_t)1 << 30) return fail(MTC_E_SHAPE, "M=%d gives too many tiles", M);
-  const int tiles_per_xcd = (int)((n_tiles + kXcds - 1) / kXcds);
-  const void* fn = cell_format(d) == kCellFp32   ? reinterpret_cast<const void*>(&k_gemm_f32<kCellFp32>)
-                   : cell_format(d) == kCellCols ? reinterpret_cast<const void*>(&k_gemm_f32<kCellCols>)
-                                                 : reinterpret_cast<const void*>(&k_gemm_f32<kCellBf16>);
-  hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytesF32);
-  if (e != hipSuccess) return fail(MTC_E_LAUNCH, "hipFuncSetAttribute: %s", hipGetErrorString(e));
-  int nrt = n_row_tiles, tpx = tiles_per_xcd, spp = p.per;
-  void* args[] = {const_cast<mtc_tile_desc*>(d), &xa, &lda, &Y, &ldy, &M, &nrt, &tpx, &spp, &part};
-  e = hipLaunchKernel(fn, dim3(tiles_per_xcd * kXcds, p.splits), dim3(kThreads), args, kLdsBytesF32, st);
-  if (e != hipSuccess) return fail(MTC_E_LAUNCH, "k_gemm_f32 launch: %s", hipGetErrorString(e));
-  rc = check_launch("k_gemm_f32");
+  switch (cell_format(d)) {
+    case kCellFp32: rc = launch_f32<kCellFp32>(d, p, xa, lda, Y, ldy, M, part, st); break;
+    case kCellCols: rc = launch_f32<kCellCols>(d, p, xa, lda, Y, ldy, M, part, st); break;
+    default: rc = launch_f32<kCellBf16>(d, p, xa, lda, Y, ldy, M, part, st);
+  }
   if (rc || p.splits == 1) return rc;
   hipLaunchKernelGGL(k_splitk_reduce<MTC_DTYPE_F32>, dim3((unsigned)reduce_blocks(M, d->N, d->col_perm != nullptr)),
                      dim3(kReduceThreads), 0, st, part, p.splits, M, d->N, d->col_perm, Y, ldy);

@@ -617,10 +617,7 @@ def _kernel_layout(X):
 
 def _gemm_f32(B: "MTCMatrix", Xf, dev):
     """fp32 Y = Xf @ W_hat: the decode kernels over the panel stream up to F32_DECODE_MAX_M rows,
-    the fp32 matrix-core tile path above. The tile path is faster from 16 rows on (c2: M = 16 23.0
-    against 24.0 µs, M = 64 52 against 73 µs, M = 256 176 against 276 µs) but its cell
-    descriptors and split-K partials move 40 MB per call at c2 M = 16 against 14 MB for the
-    decode path, so the decode path keeps M <= 16."""
+    the fp32 matrix-core tile path above (4096 x 4096 QT-P, M = 16: 24 us on either; M = 64: 33 against 73)."""
     M = Xf.shape[0]
     if M > F32_DECODE_MAX_M:
         if Xf.stride(0) % 4 or Xf.data_ptr() % 16:   # the tile kernel reads rows in 16-byte pieces

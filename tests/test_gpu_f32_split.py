@@ -1,0 +1,94 @@
+"""fp32 results on the bf16 matrix cores (mtc_gemm_f32, k_gemm_f32; run on an MI355X): X and the
+weights cut into bf16 planes, at every tile height's edges, and values that have no such planes."""
+
+import numpy as np
+import pytest
+
+from oracle import mtc_oracle as O
+from tensorpack_amd.core.allocation import rd_allocate
+from tensorpack_amd.core.permutation import PermutedQuadtreeRD
+from tensorpack_amd.core.quadtree import QuadtreeRD
+from tensorpack_amd.kernels.gemm import MTCMatrix
+
+from conftest import outlier_matrix
+
+pytestmark = pytest.mark.gpu
+
+# (K, N): a partial last K-step and column tile; many K-steps (split K, several per block)
+SHAPES = {"ragged": (992, 288), "deep": (4096, 544)}
+
+
+@pytest.fixture(scope="module")
+def mats():
+    out = {}
+    for shape, (K, N) in SHAPES.items():
+        W = outlier_matrix(K + N, K, N)
+        h = np.exp(np.random.RandomState(K).randn(K))
+        for form, bits in (("qt", 4.0), ("qtp", 3.5), ("p16", 11.0)):
+            a = (PermutedQuadtreeRD if form == "qtp" else QuadtreeRD)(W, h, (32, 16, 8, 4)).select(bits)
+            i = getattr(a, "inner", a)
+            if form == "qtp":
+                W_hat = O.permuted_qt_dequant(W, a.row_perm, a.col_perm, i.sizes, i.leaf, i.modes, i.scales)
+            else:
+                W_hat = O.qt_dequant(W, i.sizes, i.leaf, i.modes, i.scales)
+            out[shape, form] = MTCMatrix.from_quadtree(a, W), W_hat
+        al = rd_allocate(W, 4.5, None, 32)
+        out[shape, "uniform"] = (MTCMatrix.from_allocation(W, al.modes, al.scales, 32),
+                                 O.uniform_to_array(W, al.modes, al.scales, 32))
+    return out
+
+
+def _tol(K):
+    # each output: 6 MFMA sums per 16 rows of K, each rounded once to fp32 (a random walk of half-ulp
+    # steps on the running sum), and the plane products left out, below 2^-24 of their product
+    return (np.sqrt(6 * K / 16) + 2) * 2.0 ** -25
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+@pytest.mark.parametrize("form", ["qt", "qtp", "p16", "uniform"])
+def test_f32_tiles_at_every_height(gpu, mats, shape, form):
+    import torch
+    m, W_hat = mats[shape, form]
+    K = W_hat.shape[0]
+    t = m.device_tiles(gpu)
+    for M in (1, 17, 31, 32, 33, 64, 65, 100, 128, 129, 250):
+        print("f32 split", shape, form, M, flush=True)
+        X = (np.random.RandomState(M).randn(M, K) * np.exp(3 * np.random.RandomState(K).randn(K))).astype(np.float32)
+        Y = t.gemm_f32(torch.from_numpy(X).to(gpu)).cpu().numpy()
+        err = O.relative_frobenius_error(O.qt_gemm_f64(X, W_hat), Y)
+        assert err <= _tol(K), (M, err)
+
+
+@pytest.mark.parametrize("form", ["qt", "qtp", "uniform"])
+@pytest.mark.parametrize("M", [20, 64, 100])
+def test_f32_tiles_infinities_nan_and_range(gpu, mats, form, M):
+    """Infinities and NaN go where the fp64 product has them, the other rows keep their values; finite
+    values near the end of fp32's range (bf16's rounding would make them infinite) give finite results,
+    and subnormal ones are not worse than an absolute 2^-126 a product."""
+    import torch
+    m, W_hat = mats["ragged", form]
+    K = W_hat.shape[0]
+    t = m.device_tiles(gpu)
+    X = np.random.RandomState(M).randn(M, K).astype(np.float32)
+    Z = X.copy()
+    Z[3, 5], Z[7, 100], Z[M - 1, K - 1] = np.inf, np.nan, -np.inf
+    print("f32 split non-finite", form, M, flush=True)
+    Y = t.gemm_f32(torch.from_numpy(Z).to(gpu)).cpu().numpy()
+    with np.errstate(invalid="ignore"):
+        ref = Z.astype(np.float64) @ W_hat.astype(np.float64)
+    assert np.array_equal(np.isnan(Y), np.isnan(ref)) and np.array_equal(np.isinf(Y), np.isinf(ref))
+    assert np.array_equal(np.sign(Y[np.isinf(Y)]), np.sign(ref[np.isinf(ref)]))
+    rows = np.setdiff1d(np.arange(M), [3, 7, M - 1])
+    assert O.relative_frobenius_error(ref[rows], Y[rows]) <= np.sqrt(K) * 2.0 ** -25    # an fma chain of K steps
+    big = np.zeros((M, K), np.float32)
+    big[np.arange(M), np.arange(M)] = np.float32(3.4e38)
+    small = np.abs(W_hat[:M]).max(axis=1, keepdims=True) < 0.99
+    Yb = t.gemm_f32(torch.from_numpy(big).to(gpu)).cpu().numpy()
+    with np.errstate(over="ignore"):
+        want = (big.astype(np.float64) @ W_hat.astype(np.float64)).astype(np.float32)
+    sel = small & np.isfinite(want)
+    assert sel.any() and np.allclose(Yb[sel], want[sel], rtol=2.0 ** -22, atol=0)
+    tiny = (X * 1e-38).astype(np.float32)
+    Yt = t.gemm_f32(torch.from_numpy(tiny).to(gpu)).cpu().numpy().astype(np.float64)
+    ref = tiny.astype(np.float64) @ W_hat.astype(np.float64)
+    assert np.abs(Yt - ref).max() <= K * 2.0 ** -126 * np.abs(W_hat).max()
