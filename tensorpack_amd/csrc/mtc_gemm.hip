@@ -8,9 +8,7 @@
 //   k_gemm_tile : one 256 x 256 output tile per block, K in steps of 64. Warp-specialized:
 //                 8 consumer waves (2 x 4 of 128 x 64 outputs) copy X tiles straight
 //                 into LDS (buffer loads with the LDS destination, two steps ahead into
-//                 three A buffers; unpermuted fp32 X in tiles of 64 or 128 rows goes
-//                 through registers instead, rounded to bf16 on the way) and issue the
-//                 MFMAs; 4 producer waves (one per SIMD)
+//                 three A buffers) and issue the MFMAs; 4 producer waves (one per SIMD)
 //                 decode step k+1's weight cells from registers into the other of two B
 //                 buffers and load step k+2's cell payload. Tiles use an XOR swizzle of
 //                 16-byte segments; one LDS-only barrier per step (global loads stay in
@@ -19,6 +17,7 @@
 //                 W_hat once into bf16 and multiplies it with a plain hipBLASLt GEMM instead
 //                 (the tile kernel would decode each weight step once per row tile).
 //   k_tile_dequant_rows : W_hat in fp32 rows (mtc_tile_dequant).
+//   k_gemm_tile_short : the prefill in row tiles of 32, 64 or 128 rows, for few rows (mtc_gemm_short.h).
 //   k_gemm_f32  : fp32 results (mtc_gemm_f32), from bf16 planes of X and W_hat (mtc_gemm_short.h).
 //
 // Reference behaviour: mtc/kernels/gemm.py:124-210 (block loop: skip P0 blocks,
@@ -413,18 +412,14 @@ __device__ __forceinline__ void tile_producers(const mtc_tile_desc& d, const int
 }
 
 // One output tile block of matrix `d`: output tile (rt, ct), K split by.
-// TM: output rows of the block (256, or 128 / 64 for short X, whose full-height tiles are too
-// few to fill the chip). The 8 consumer waves are 2 x 4: TM / 2 rows x 64 columns each.
-// Xv: bf16 X (copied into LDS as is), or with kXF fp32 X in original row order, which the
-// consumers round to bf16 on the way into LDS (tiles of at most 128 rows, whose consumers have
-// the registers to hold two steps of X in flight).
-template <int kCF, int kYDT, int TM = kTM, bool kXF = false>
+// The 8 consumer waves are 2 x 4: 128 rows x 64 columns each. (Short X, whose 256-row tiles are too few
+// to fill the chip: gemm_short_block.)
+template <int kCF, int kYDT>
 __device__ __forceinline__ void gemm_tile_block(const mtc_tile_desc& d, const int rt, const int ct, const int by,
                                                 const void* __restrict__ Xv, int64_t ldx, void* __restrict__ Y,
                                                 int64_t ldy, int M, int steps_per_split, float* __restrict__ part) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
-  static_assert(TM == 256 || TM == 128 || TM == 64, "row tiles of 256, 128 or 64 rows");
-  static_assert(!kXF || TM <= 128, "fp32 X is rounded by the consumers of tiles of at most 128 rows");
+  constexpr int TM = kTM;
   constexpr int DMA = TM / 8 / kConsumerWaves;             // 1 KiB (8-row) A copies per consumer wave
   constexpr int RW = TM / 2, RI = RW / 32;                 // rows per consumer wave, 32-row MFMA blocks
 
@@ -485,82 +480,35 @@ __device__ __forceinline__ void gemm_tile_block(const mtc_tile_desc& d, const in
       }
     };
 
-    if constexpr (!kXF) {
-      const __bf16* X = reinterpret_cast<const __bf16*>(Xv);
-      const u32x4_t x_r = buffer_rsrc(X + (int64_t)m0 * ldx, (uint32_t)(TM * ldx * 2));
-      auto copy_a = [&](int s) __attribute__((always_inline)) {
-        const uint32_t buf = lds0 + (uint32_t)(s % kABufs) * kTileBytes;
-        const uint32_t kb = (uint32_t)((kb0 + s) * kTK) * 2;
+    const __bf16* X = reinterpret_cast<const __bf16*>(Xv);
+    const u32x4_t x_r = buffer_rsrc(X + (int64_t)m0 * ldx, (uint32_t)(TM * ldx * 2));
+    auto copy_a = [&](int s) __attribute__((always_inline)) {
+      const uint32_t buf = lds0 + (uint32_t)(s % kABufs) * kTileBytes;
+      const uint32_t kb = (uint32_t)((kb0 + s) * kTK) * 2;
 #pragma unroll
-        for (int i = 0; i < DMA; ++i)
-          dma16(x_r, a_in(s, i) ? a_off[i] * 2 + kb : kOutOfRange,
-                __builtin_amdgcn_readfirstlane(buf + (uint32_t)(DMA * wave + i) * 1024u));
-      };
-      copy_a(0);
-      if (nks > 1) {
-        copy_a(1);
-        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(DMA) : "memory");   // step 0's copies done
+      for (int i = 0; i < DMA; ++i)
+        dma16(x_r, a_in(s, i) ? a_off[i] * 2 + kb : kOutOfRange,
+              __builtin_amdgcn_readfirstlane(buf + (uint32_t)(DMA * wave + i) * 1024u));
+    };
+    copy_a(0);
+    if (nks > 1) {
+      copy_a(1);
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(DMA) : "memory");   // step 0's copies done
+    } else {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    }
+    lds_barrier();                                       // step 0 staged
+    for (int ks = 0; ks < nks; ++ks) {
+      const bool ahead = ks + 2 < nks;
+      if (ahead) copy_a(ks + 2);                         // into the buffer step ks-1 used
+      mfma_step(ks);
+      // step ks+1's copies (issued a step ago) must have landed before the barrier
+      if (ahead) {
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(DMA) : "memory");
       } else {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       }
-      lds_barrier();                                       // step 0 staged
-      for (int ks = 0; ks < nks; ++ks) {
-        const bool ahead = ks + 2 < nks;
-        if (ahead) copy_a(ks + 2);                         // into the buffer step ks-1 used
-        mfma_step(ks);
-        // step ks+1's copies (issued a step ago) must have landed before the barrier
-        if (ahead) {
-          asm volatile("s_waitcnt vmcnt(%0)" ::"n"(DMA) : "memory");
-        } else {
-          asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        }
-        lds_barrier();                                     // buffers of step ks free, step ks+1 staged
-      }
-    } else {
-      // fp32 X: the lane reads its segment's 8 floats (two 16-byte loads; zeros past M and K),
-      // rounds them to bf16 as the staging kernels do (pk_bf16) and stores its slot. Step s + 2's
-      // loads go out before step s's MFMAs into the registers step s held; step s + 1's values
-      // are stored after them, into the buffer step s - 2 used.
-      const float* Xf = reinterpret_cast<const float*>(Xv);
-      const __amdgpu_buffer_rsrc_t xf_r = buffer_of(Xf + (int64_t)m0 * ldx, (int64_t)TM * ldx * 4);
-      typedef u32x4_t XRegs[DMA][2];
-      auto load_x = [&](int s, XRegs& r) __attribute__((always_inline)) {
-        const uint32_t kb = (uint32_t)((kb0 + s) * kTK) * 4;
-#pragma unroll
-        for (int i = 0; i < DMA; ++i) {
-          const bool in = a_in(s, i);
-          r[i][0] = __builtin_amdgcn_raw_buffer_load_b128(xf_r, in ? a_off[i] * 4 + kb : kOutOfRange, 0, 0);
-          r[i][1] = __builtin_amdgcn_raw_buffer_load_b128(xf_r, in ? a_off[i] * 4 + kb + 16 : kOutOfRange, 0, 0);
-        }
-      };
-      auto store_x = [&](int s, const XRegs& r) __attribute__((always_inline)) {
-        unsigned char* buf = lds + (s % kABufs) * kTileBytes;
-#pragma unroll
-        for (int i = 0; i < DMA; ++i) {
-          const u32x4_t lo = r[i][0], hi = r[i][1];
-          const u32x4_t o{pk_bf16(__uint_as_float(lo.x), __uint_as_float(lo.y)),
-                          pk_bf16(__uint_as_float(lo.z), __uint_as_float(lo.w)),
-                          pk_bf16(__uint_as_float(hi.x), __uint_as_float(hi.y)),
-                          pk_bf16(__uint_as_float(hi.z), __uint_as_float(hi.w))};
-          *reinterpret_cast<u32x4_t*>(buf + (DMA * wave + i) * 1024 + 16 * lane) = o;
-        }
-      };
-      XRegs ra, rb;
-      load_x(0, ra);
-      if (nks > 1) load_x(1, rb);
-      store_x(0, ra);
-      lds_barrier();                                       // step 0 staged
-      // cur: step ks's registers (stored a step ago), nxt: step ks + 1's
-      auto body = [&](int ks, XRegs& cur, const XRegs& nxt) __attribute__((always_inline)) {
-        if (ks + 2 < nks) load_x(ks + 2, cur);
-        mfma_step(ks);
-        if (ks + 1 < nks) store_x(ks + 1, nxt);
-        lds_barrier();                                     // buffers of step ks free, step ks+1 staged
-      };
-      for (int ks = 0; ks < nks; ks += 2) {
-        body(ks, ra, rb);
-        if (ks + 1 < nks) body(ks + 1, rb, ra);
-      }
+      lds_barrier();                                     // buffers of step ks free, step ks+1 staged
     }
 
     // epilogue: C element e of lane l is row (e/4)*8 + (l/32)*4 + e%4, column l%32.
@@ -593,19 +541,28 @@ __device__ __forceinline__ void gemm_tile_block(const mtc_tile_desc& d, const in
   tile_producers<kCF>(d, ct, kb0, nks, lds + kABufs * kTileBytes, tid - 64 * kConsumerWaves);
 }
 
-// One output tile block of matrix `d`: output tile (rt, ct) of TM rows, K split by; X is bf16,
-// or fp32 with kXF.
-template <int kCF, int kYDT, int TM, bool kXF = false>
+// One output tile block of matrix `d`: output tile (rt, ct) of 256 rows, K split by; X is bf16.
+template <int kCF, int kYDT>
 __global__ __launch_bounds__(kThreads) void k_gemm_tile(const mtc_tile_desc d, const void* __restrict__ X,
                                                         int64_t ldx, void* __restrict__ Y, int64_t ldy, int M,
                                                         int n_row_tiles, int tiles_per_xcd, int steps_per_split,
                                                         float* __restrict__ part) {
   int rt, ct;
   if (!tile_of_block((int)blockIdx.x, n_row_tiles, d.n_col_tiles, tiles_per_xcd, d.col_perm && !part, rt, ct)) return;
-  gemm_tile_block<kCF, kYDT, TM, kXF>(d, rt, ct, (int)blockIdx.y, X, ldx, Y, ldy, M, steps_per_split, part);
+  gemm_tile_block<kCF, kYDT>(d, rt, ct, (int)blockIdx.y, X, ldx, Y, ldy, M, steps_per_split, part);
 }
 
 #include "mtc_gemm_short.h"
+
+// The same in tiles of TM <= 128 rows, for bf16 or fp32 (kXRound) X.
+template <int kCF, int kYDT, int XM, int TM>
+__global__ __launch_bounds__((ShortTile<XM, TM>::threads)) void k_gemm_tile_short(
+    const mtc_tile_desc d, const void* __restrict__ X, int64_t ldx, void* __restrict__ Y, int64_t ldy, int M,
+    int n_row_tiles, int tiles_per_xcd, int steps_per_split, float* __restrict__ part) {
+  int rt, ct;
+  if (!tile_of_block((int)blockIdx.x, n_row_tiles, d.n_col_tiles, tiles_per_xcd, d.col_perm && !part, rt, ct)) return;
+  gemm_short_block<kCF, kYDT, XM, TM>(d, rt, ct, (int)blockIdx.y, X, ldx, Y, ldy, M, steps_per_split, part);
+}
 
 // fp32 results (mtc_gemm_f32): Y = X * W_hat with fp32 X and the exact W_hat.
 template <int kCF, int TM>
@@ -836,18 +793,31 @@ struct GemmGroup {
   int start[kMaxGroup + 1];
 };
 
-template <int kCF, int kYDT, int TM>
-__global__ __launch_bounds__(kThreads) void k_gemm_tile_group(const GemmGroup g, int M, int n_row_tiles) {
-  int i = 0;
+// Block bx, split by of a group: its member and output tile; false for a block with no work.
+__device__ __forceinline__ bool group_tile(const GemmGroup& g, int bx, int by, int n_row_tiles, int& i, int& rt, int& ct) {
+  i = 0;
 #pragma unroll
-  for (int k = 1; k < kMaxGroup; ++k) i += (int)blockIdx.x >= g.start[k];
-  if ((int)blockIdx.y >= g.splits[i]) return;               // this member has fewer K splits
-  int rt, ct;
-  if (!tile_of_block((int)blockIdx.x - g.start[i], n_row_tiles, g.d[i].n_col_tiles, g.tiles_per_xcd[i],
-                     g.d[i].col_perm && !g.part[i], rt, ct))
-    return;
-  gemm_tile_block<kCF, kYDT, TM>(g.d[i], rt, ct, (int)blockIdx.y, g.X[i], g.ldx[i], g.Y[i], g.ldy[i], M,
-                                 g.steps_per_split[i], g.part[i]);
+  for (int k = 1; k < kMaxGroup; ++k) i += bx >= g.start[k];
+  if (by >= g.splits[i]) return false;                      // this member has fewer K splits
+  return tile_of_block(bx - g.start[i], n_row_tiles, g.d[i].n_col_tiles, g.tiles_per_xcd[i],
+                       g.d[i].col_perm && !g.part[i], rt, ct);
+}
+
+template <int kCF, int kYDT>
+__global__ __launch_bounds__(kThreads) void k_gemm_tile_group(const GemmGroup g, int M, int n_row_tiles) {
+  int i, rt, ct;
+  if (!group_tile(g, (int)blockIdx.x, (int)blockIdx.y, n_row_tiles, i, rt, ct)) return;
+  gemm_tile_block<kCF, kYDT>(g.d[i], rt, ct, (int)blockIdx.y, g.X[i], g.ldx[i], g.Y[i], g.ldy[i], M,
+                             g.steps_per_split[i], g.part[i]);
+}
+
+template <int kCF, int kYDT, int TM>
+__global__ __launch_bounds__((ShortTile<kXBf16, TM>::threads)) void k_gemm_tile_short_group(const GemmGroup g, int M,
+                                                                                           int n_row_tiles) {
+  int i, rt, ct;
+  if (!group_tile(g, (int)blockIdx.x, (int)blockIdx.y, n_row_tiles, i, rt, ct)) return;
+  gemm_short_block<kCF, kYDT, kXBf16, TM>(g.d[i], rt, ct, (int)blockIdx.y, g.X[i], g.ldx[i], g.Y[i], g.ldy[i], M,
+                                          g.steps_per_split[i], g.part[i]);
 }
 
 // Xp[m, k] = bf16(X[m, row_perm[k]]) (identity without a permutation); 8 outputs per thread.
@@ -1030,14 +1000,25 @@ struct GemmBatchItem {
 
 constexpr uint32_t kNoItem = 0xFFFFFFFFu;   // a block table entry with no work
 
-template <int kCF, int kYDT, int TM>
+template <int kCF, int kYDT>
 __global__ __launch_bounds__(kThreads) void k_gemm_tile_batch(const GemmBatchItem* __restrict__ items,
                                                               const uint2* __restrict__ blocks, int M) {
   const uint2 e = blocks[blockIdx.x];
   if (e.x == kNoItem) return;                               // padding of an XCD's block list
   const GemmBatchItem& it = items[e.x];
-  gemm_tile_block<kCF, kYDT, TM>(it.d, (int)(e.y & 0xFFFu), (int)((e.y >> 12) & 0xFFFu), (int)(e.y >> 24), it.X,
-                                 it.ldx, it.Y, it.ldy, M, it.steps_per_split, it.splits > 1 ? it.part : nullptr);
+  gemm_tile_block<kCF, kYDT>(it.d, (int)(e.y & 0xFFFu), (int)((e.y >> 12) & 0xFFFu), (int)(e.y >> 24), it.X, it.ldx,
+                             it.Y, it.ldy, M, it.steps_per_split, it.splits > 1 ? it.part : nullptr);
+}
+
+template <int kCF, int kYDT, int TM>
+__global__ __launch_bounds__((ShortTile<kXBf16, TM>::threads)) void k_gemm_tile_short_batch(
+    const GemmBatchItem* __restrict__ items, const uint2* __restrict__ blocks, int M) {
+  const uint2 e = blocks[blockIdx.x];
+  if (e.x == kNoItem) return;
+  const GemmBatchItem& it = items[e.x];
+  gemm_short_block<kCF, kYDT, kXBf16, TM>(it.d, (int)(e.y & 0xFFFu), (int)((e.y >> 12) & 0xFFFu), (int)(e.y >> 24),
+                                          it.X, it.ldx, it.Y, it.ldy, M, it.steps_per_split,
+                                          it.splits > 1 ? it.part : nullptr);
 }
 
 __global__ __launch_bounds__(kStageThreads) void k_stage_x_batch(const GemmBatchItem* __restrict__ items,
@@ -1089,14 +1070,15 @@ bool needs_staging(const mtc_tile_desc* d, int x_dtype) { return d->row_perm || 
 
 constexpr int kFillCUs = 256;             // blocks that fill the chip (one tile block per CU)
 constexpr int kMinStepsPerSplit = 2;
-constexpr double kReduceBytesPerUs = 4.0e6;   // split-K partials written + read, bytes per microsecond
+constexpr double kReduceBytesPerUs = 5.0e6;   // split-K partials written + read, bytes per microsecond
 constexpr double kReduceLaunchUs = 3.0;   // the reduction pass's own launch
 
-// Time of one K-step of a tile block by its row-tile height: 256 rows 1.9-2.4 us. Shorter
-// tiles read less X from LDS per step but decode the same 64 x 256 weight cells and keep
-// the block's fixed costs; timed at 4096 x 4096, M = 256 with forced plans, relative to 256
-// rows: 128 rows 0.79, 64 rows 0.68 (with their fixed costs) of the step time.
-inline double step_us(int tm) { return tm == 256 ? 2.0 : tm == 128 ? 1.58 : 1.36; }
+// Time of one K-step of a tile block by its row-tile height, and of its launch to the first step's data
+// (kBlockUs). 256 rows (k_gemm_tile) 1.9-2.4 us; the short kernels at 4096 x 4096 in 32, 64 and 128 rows
+// without a K split: 57.8, 67.6 and 85.8 us for 64 steps. The reduction: 4.4 us with 2 splits, 8.4 with
+// 8 (M = 100, 64-row tiles).
+constexpr double kBlockUs = 4.0;
+inline double step_us(int tm) { return tm == 256 ? 2.0 : tm == 128 ? 1.28 : tm == 64 ? 0.97 : 0.85; }
 
 struct TilePlan {
   int tm;        // output rows per tile block
@@ -1105,26 +1087,29 @@ struct TilePlan {
 };
 
 // Tile height and K split of one call: with M rows in tiles of 256 when those fill the chip;
-// otherwise the height (256, or for M <= 256 also 128 or 64) and split count (at most enough
-// blocks to fill the chip, at least kMinStepsPerSplit K-steps per split) that minimise the
-// estimated time: K-steps per block, rounds of blocks past one per CU, and the split-K
-// partial traffic (written by the tile blocks, read by the reduction).
+// otherwise the height (256, or for M <= 256 also 128, 64 or for M <= 32 32) and split count (at least
+// kMinStepsPerSplit K-steps per split) that minimise the estimated time: K-steps per block, rounds of
+// blocks past one per CU, and the split-K partial traffic (written by the tile blocks, read by the
+// reduction). Rounds are counted on the fullest XCD: 22 column tiles are 3 on seven XCDs and 1 on the
+// eighth, and 11 splits of them, 242 blocks, are two rounds there (2072 x 5472 uniform, M = 40: 20.9 us
+// with 11 splits, 15.2 with 7 to 8, 15.5 with 6).
 TilePlan tile_plan(const mtc_tile_desc* d, int M) {
   const int64_t full = (int64_t)((M + kTM - 1) / kTM) * d->n_col_tiles;
   if (full >= kFillCUs) return {kTM, 1, d->n_ksteps};
   const double split_bytes = 2.0 * 4.0 * (double)M * d->N;     // one partial, written and read
   TilePlan best{kTM, 1, d->n_ksteps};
   double best_t = 1e300;
-  for (int tm : {256, 128, 64}) {
+  for (int tm : {256, 128, 64, 32}) {
     if (tm < kTM && M > kTM) break;                         // shorter tiles timed for M <= 256 only
+    if (tm == 32 && M > 32) break;                          // (two 32-row tiles decode every weight twice)
     const int64_t n_tiles = (int64_t)((M + tm - 1) / tm) * d->n_col_tiles;
     int max_s = n_tiles >= kFillCUs ? 1 : (int)((kFillCUs + n_tiles - 1) / n_tiles);
     max_s = std::max(1, std::min(max_s, d->n_ksteps / kMinStepsPerSplit));
     for (int s = 1; s <= max_s; ++s) {
       const int per = (d->n_ksteps + s - 1) / s;
       const int s_eff = (d->n_ksteps + per - 1) / per;
-      const double rounds = std::ceil((double)(n_tiles * s_eff) / kFillCUs);
-      const double t = rounds * per * step_us(tm) +
+      const double rounds = std::ceil((double)((n_tiles + kXcds - 1) / kXcds * s_eff) / (kFillCUs / kXcds));
+      const double t = rounds * (per * step_us(tm) + kBlockUs) +
                        (s_eff > 1 ? s_eff * split_bytes / kReduceBytesPerUs + kReduceLaunchUs : 0.0);
       if (t < best_t) {
         best_t = t;
@@ -1155,13 +1140,22 @@ size_t partial_bytes(const mtc_tile_desc* d, int M) {
   return splits > 1 ? (size_t)splits * M * d->N * 4 : 0;
 }
 
-// fp32 X that the tile kernel's consumers round to bf16 themselves, with no staging launch:
+// fp32 X that the short kernel rounds to bf16 itself, with no staging launch:
 // no row permutation, tiles of at most 128 rows, 16-byte aligned rows, and tile offsets within
 // 32 bits. The sums are those of the staged call (same bf16 values, same kernel otherwise).
 bool fused_x(const mtc_tile_desc* d, const void* X, int x_dtype, int64_t ldx, int M) {
   return x_dtype == MTC_DTYPE_F32 && !d->row_perm && cell_format(d) != kCellCols && tile_plan(d, M).tm <= 128 &&
          ldx % 4 == 0 && (reinterpret_cast<uintptr_t>(X) & 15) == 0 && ldx < ((int64_t)1 << 31) / (4 * kTM);
 }
+
+// LDS and threads of a tile block by its row-tile height: k_gemm_tile's, or the short kernels'.
+int tile_lds_bytes(int tm) {
+  return tm == 256   ? kLdsBytes
+         : tm == 128 ? ShortTile<kXBf16, 128>::lds_bytes
+         : tm == 64  ? ShortTile<kXBf16, 64>::lds_bytes
+                     : ShortTile<kXBf16, 32>::lds_bytes;
+}
+int tile_threads(int tm) { return tm == 256 ? kThreads : ShortTile<kXBf16, 32>::threads; }
 
 template <int kCF, int kYDT>
 int launch_tile(const mtc_tile_desc* d, const void* X, int64_t ldx, void* Y, int64_t ldy, int M, float* part,
@@ -1173,17 +1167,20 @@ int launch_tile(const mtc_tile_desc* d, const void* X, int64_t ldx, void* Y, int
     return fail(MTC_E_SHAPE, "ldx=%lld too large for 32-bit X tile offsets", (long long)ldx);
   const TilePlan p = tile_plan(d, M);
   if (xf && p.tm > 128) return fail(MTC_E_SHAPE, "fp32 X is read in place by tiles of at most 128 rows only");
-  const void* fn = p.tm == 256 ? reinterpret_cast<const void*>(&k_gemm_tile<kCF, kYDT, 256>)
-                   : p.tm == 128 ? reinterpret_cast<const void*>(&k_gemm_tile<kCF, kYDT, 128>)
-                                 : reinterpret_cast<const void*>(&k_gemm_tile<kCF, kYDT, 64>);
+  const void* fn = p.tm == 256   ? reinterpret_cast<const void*>(&k_gemm_tile<kCF, kYDT>)
+                   : p.tm == 128 ? reinterpret_cast<const void*>(&k_gemm_tile_short<kCF, kYDT, kXBf16, 128>)
+                   : p.tm == 64  ? reinterpret_cast<const void*>(&k_gemm_tile_short<kCF, kYDT, kXBf16, 64>)
+                                 : reinterpret_cast<const void*>(&k_gemm_tile_short<kCF, kYDT, kXBf16, 32>);
   if constexpr (kCF != kCellCols) {
     if (xf)
-      fn = p.tm == 128 ? reinterpret_cast<const void*>(&k_gemm_tile<kCF, kYDT, 128, true>)
-                       : reinterpret_cast<const void*>(&k_gemm_tile<kCF, kYDT, 64, true>);
+      fn = p.tm == 128  ? reinterpret_cast<const void*>(&k_gemm_tile_short<kCF, kYDT, kXRound, 128>)
+           : p.tm == 64 ? reinterpret_cast<const void*>(&k_gemm_tile_short<kCF, kYDT, kXRound, 64>)
+                        : reinterpret_cast<const void*>(&k_gemm_tile_short<kCF, kYDT, kXRound, 32>);
   } else if (xf) {
     return fail(MTC_E_SHAPE, "fp32 X is not read in place for gathered-column streams");
   }
-  hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes);
+  const int lds = tile_lds_bytes(p.tm), threads = tile_threads(p.tm);
+  hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
   if (e != hipSuccess) return fail(MTC_E_LAUNCH, "hipFuncSetAttribute: %s", hipGetErrorString(e));
   const int n_row_tiles = (M + p.tm - 1) / p.tm;
   const int64_t n_tiles = (int64_t)n_row_tiles * d->n_col_tiles;
@@ -1194,9 +1191,9 @@ int launch_tile(const mtc_tile_desc* d, const void* X, int64_t ldx, void* Y, int
   int nrt = n_row_tiles, tpx = tiles_per_xcd, spp = per;
   const dim3 grid(tiles_per_xcd * kXcds, splits);
   void* args[] = {const_cast<mtc_tile_desc*>(d), &X, &ldx, &Y, &ldy, &M, &nrt, &tpx, &spp, &pt};
-  e = hipLaunchKernel(fn, grid, dim3(kThreads), args, kLdsBytes, st);
-  if (e != hipSuccess) return fail(MTC_E_LAUNCH, "k_gemm_tile launch: %s", hipGetErrorString(e));
-  int rc = check_launch("k_gemm_tile");
+  e = hipLaunchKernel(fn, grid, dim3(threads), args, lds, st);
+  if (e != hipSuccess) return fail(MTC_E_LAUNCH, "prefill tile kernel launch: %s", hipGetErrorString(e));
+  int rc = check_launch("prefill tile kernel");
   if (rc || splits == 1) return rc;
   hipLaunchKernelGGL(k_splitk_reduce<kYDT>, dim3((unsigned)reduce_blocks(M, d->N, d->col_perm != nullptr)),
                      dim3(kReduceThreads), 0, st, part, splits, M, d->N, d->col_perm, Y, ldy);
@@ -1456,21 +1453,20 @@ int launch_tile_group(GemmGroup& g, int n, int M, int tm, const ReduceGroup& rg,
   if ((size_t)kLdsBytes > mtc::host::device_lds_limit())
     return fail(MTC_E_SHAPE, "prefill kernel needs %d B of LDS per block, device has %zu", kLdsBytes,
                 mtc::host::device_lds_limit());
-  const void* fn = tm == 256 ? reinterpret_cast<const void*>(&k_gemm_tile_group<kCF, kYDT, 256>)
-                   : tm == 128 ? reinterpret_cast<const void*>(&k_gemm_tile_group<kCF, kYDT, 128>)
-                               : reinterpret_cast<const void*>(&k_gemm_tile_group<kCF, kYDT, 64>);
-  hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes);
+  const void* fn = tm == 256   ? reinterpret_cast<const void*>(&k_gemm_tile_group<kCF, kYDT>)
+                   : tm == 128 ? reinterpret_cast<const void*>(&k_gemm_tile_short_group<kCF, kYDT, 128>)
+                   : tm == 64  ? reinterpret_cast<const void*>(&k_gemm_tile_short_group<kCF, kYDT, 64>)
+                               : reinterpret_cast<const void*>(&k_gemm_tile_short_group<kCF, kYDT, 32>);
+  const int lds = tile_lds_bytes(tm);
+  hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
   if (e != hipSuccess) return fail(MTC_E_LAUNCH, "hipFuncSetAttribute: %s", hipGetErrorString(e));
-  const int n_row_tiles = (M + tm - 1) / tm;
+  int n_row_tiles = (M + tm - 1) / tm;
   int max_splits = 1;
   for (int i = 0; i < n; ++i) max_splits = std::max(max_splits, g.splits[i]);
   const dim3 grid(g.start[n], max_splits);
-  if (tm == 256)
-    hipLaunchKernelGGL((k_gemm_tile_group<kCF, kYDT, 256>), grid, dim3(kThreads), kLdsBytes, st, g, M, n_row_tiles);
-  else if (tm == 128)
-    hipLaunchKernelGGL((k_gemm_tile_group<kCF, kYDT, 128>), grid, dim3(kThreads), kLdsBytes, st, g, M, n_row_tiles);
-  else
-    hipLaunchKernelGGL((k_gemm_tile_group<kCF, kYDT, 64>), grid, dim3(kThreads), kLdsBytes, st, g, M, n_row_tiles);
+  void* args[] = {&g, &M, &n_row_tiles};
+  e = hipLaunchKernel(fn, grid, dim3(tile_threads(tm)), args, lds, st);
+  if (e != hipSuccess) return fail(MTC_E_LAUNCH, "k_gemm_tile_group launch: %s", hipGetErrorString(e));
   int rc = check_launch("k_gemm_tile_group");
   if (rc || n_red == 0) return rc;
   int grid_x = 1;
@@ -1740,18 +1736,18 @@ int launch_tile_batch(const GemmBatchHeader* h, const GemmBatchItem* items, cons
   if ((size_t)kLdsBytes > mtc::host::device_lds_limit())
     return fail(MTC_E_SHAPE, "prefill kernel needs %d B of LDS per block, device has %zu", kLdsBytes,
                 mtc::host::device_lds_limit());
-  const void* fn = h->tm == 256 ? reinterpret_cast<const void*>(&k_gemm_tile_batch<kCF, kYDT, 256>)
-                   : h->tm == 128 ? reinterpret_cast<const void*>(&k_gemm_tile_batch<kCF, kYDT, 128>)
-                                  : reinterpret_cast<const void*>(&k_gemm_tile_batch<kCF, kYDT, 64>);
-  hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes);
+  const void* fn = h->tm == 256   ? reinterpret_cast<const void*>(&k_gemm_tile_batch<kCF, kYDT>)
+                   : h->tm == 128 ? reinterpret_cast<const void*>(&k_gemm_tile_short_batch<kCF, kYDT, 128>)
+                   : h->tm == 64  ? reinterpret_cast<const void*>(&k_gemm_tile_short_batch<kCF, kYDT, 64>)
+                                  : reinterpret_cast<const void*>(&k_gemm_tile_short_batch<kCF, kYDT, 32>);
+  const int lds = tile_lds_bytes(h->tm);
+  hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
   if (e != hipSuccess) return fail(MTC_E_LAUNCH, "hipFuncSetAttribute: %s", hipGetErrorString(e));
   const dim3 grid((unsigned)h->n_blocks);
-  if (h->tm == 256)
-    hipLaunchKernelGGL((k_gemm_tile_batch<kCF, kYDT, 256>), grid, dim3(kThreads), kLdsBytes, st, items, blocks, h->M);
-  else if (h->tm == 128)
-    hipLaunchKernelGGL((k_gemm_tile_batch<kCF, kYDT, 128>), grid, dim3(kThreads), kLdsBytes, st, items, blocks, h->M);
-  else
-    hipLaunchKernelGGL((k_gemm_tile_batch<kCF, kYDT, 64>), grid, dim3(kThreads), kLdsBytes, st, items, blocks, h->M);
+  int M = h->M;
+  void* args[] = {&items, &blocks, &M};
+  e = hipLaunchKernel(fn, grid, dim3(tile_threads(h->tm)), args, lds, st);
+  if (e != hipSuccess) return fail(MTC_E_LAUNCH, "k_gemm_tile_batch launch: %s", hipGetErrorString(e));
   int rc = check_launch("k_gemm_tile_batch");
   if (rc || h->n_reduce == 0) return rc;
   hipLaunchKernelGGL(k_splitk_reduce_batch<kYDT>, dim3((unsigned)h->reduce_blocks_x, (unsigned)h->n_reduce),

@@ -1,12 +1,16 @@
 // Row tiles of 32, 64 or 128 rows over the tile stream (included by mtc_gemm.hip, inside its
-// namespace): fp32 results for any M (k_gemm_f32) and bf16 prefill with few rows.
+// namespace): fp32 results for any M (k_gemm_f32) and bf16 prefill with few rows (k_gemm_tile_short and its
+// group and batch kernels).
 //
 // Block = one TM x 256 output tile over a run of K-steps. Every wave decodes and every
 // wave multiplies: a thread takes one cell of a step (512 cells; half a cell where a block has 1024
 // threads), whose descriptor was loaded four steps and whose payload three steps ahead, decodes it into
 // the B tile in LDS, and after the barrier the waves run the step's MFMAs. With few rows a step's MFMAs take less time than its
 // decode and its memory latency; four waves that decode for eight that multiply (k_gemm_tile) then leave
-// most of a CU's issue slots idle.
+// most of a CU's issue slots idle. Sums run in k_gemm_tile's order: the same bits for the same K splits.
+// Measured against k_gemm_tile's blocks of 64 or 128 rows, with the plan of tile_plan, us a call: 2072 x 5472
+// uniform, M = 40: 23.0 -> 14.9; 6144 x 1024 QT, M = 160: 27.7 -> 18.9; 4096 x 4096 QT-P, M = 128: 29.0 -> 25.6;
+// M = 256 of 4096 x 4096 QT 29.1 -> 29.0 (bound by the 8 splits' partials and their reduction, about 14 us).
 //
 // fp32 results on the bf16 matrix cores. A float is cut into bf16 planes by truncation, hi + mid + lo,
 // each the upper half of what the planes before left (8 + 8 + 8 significant bits: exact). X takes
