@@ -1899,7 +1899,10 @@ int launch_f32(const mtc_tile_desc* d, const F32Plan& p, const float* X, int64_t
   hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
   if (e != hipSuccess) return fail(MTC_E_LAUNCH, "hipFuncSetAttribute: %s", hipGetErrorString(e));
   void* args[] = {const_cast<mtc_tile_desc*>(d), &X, &ldx, &Y, &ldy, &M, &nrt, &tpx, &spp, &part};
-  e = hipLaunchKernel(fn, dim3(tpx * kXcds, p.splits), dim3(ShortTile<kXSplit, 32>::threads), args, lds, st);
+  const int threads = p.tm == 128  ? ShortTile<kXSplit, 128>::threads
+                      : p.tm == 64 ? ShortTile<kXSplit, 64>::threads
+                                   : ShortTile<kXSplit, 32>::threads;
+  e = hipLaunchKernel(fn, dim3(tpx * kXcds, p.splits), dim3(threads), args, lds, st);
   if (e != hipSuccess) return fail(MTC_E_LAUNCH, "k_gemm_f32 launch: %s", hipGetErrorString(e));
   return check_launch("k_gemm_f32");
 }

@@ -13,20 +13,16 @@
 // M = 256 of 4096 x 4096 QT 29.1 -> 29.0 (bound by the 8 splits' partials and their reduction, about 14 us).
 //
 // fp32 results on the bf16 matrix cores. A float is cut into bf16 planes by truncation, hi + mid + lo,
-// each the upper half of what the planes before left (8 + 8 + 8 significant bits: exact). X takes
-// three planes; a weight code * scale with a code of at most 8 bits and a bf16 scale has at most
-// 16 significant bits and takes two, a P16 code or an fp32 scale three. The tile accumulates
-//   mid.mid + hi.lo + lo.hi + mid.hi + hi.mid + hi.hi        (weight plane . X plane)
-// in fp32: products of bf16 values are exact in fp32, and the terms left out (mid.lo, lo.mid, lo.lo)
-// are below 2^-24 of the product. v_mfma_f32_32x32x16_bf16 does 16 times the products per clock of
-// v_mfma_f32_16x16x4f32, for five or six times the number. X or weights that are not finite have no such
-// planes (inf - inf): a block that met one computes its tile again in plain fp32.
-// Measured, 4096 x 4096 QT-P @ 4.25, M = 100: 39.4 us a call against 119.8 for 16-row tiles on the fp32
-// MFMAs (which decoded every weight seven times), relative error against fp64 2.6e-7 against 5.9e-7; M = 2048
-// of QT @ 4.25: 284 us, 242 TFLOP/s of fp32 results (the library's fp32 product: 154). 128-row tiles
-// run a K-step in 1.4 us of decode and 2.2 of MFMAs at their peak rate, one after the other (two B tiles of
-// three planes do not fit the LDS); short calls are bound by launch and the descriptor -> payload chain
-// (5-9 us to the first step's data) and the split-K partials.
+// each the upper half of what the planes before left (8 + 8 + 8 significant bits: exact, mid below 2^-7 and
+// lo below 2^-15 of hi's leading bit). X takes three planes; a weight code * scale with a code of at most
+// 8 bits and a bf16 scale has at most 16 significant bits and takes two, a P16 code or an fp32 scale three.
+// Products of bf16 values are exact in fp32; all pairs of planes are multiplied but (weight . X) mid.lo, lo.mid
+// and lo.lo. v_mfma_f32_32x32x16_bf16 does 16 times the products
+// per clock of v_mfma_f32_16x16x4f32, for five or six times the number.
+//   Two accumulators: hi.hi in one, the other pairs in a second that is added at the end. In one, the small
+// pairs of a slice fall below half an ulp of a long sum of one sign, always to the same side.
+//   X or weights that are not finite have no planes (inf - inf): a block that met one computes its tile again
+// in plain fp32.
 #pragma once
 
 enum { kXBf16, kXRound, kXSplit };   // X: bf16 / fp32 rounded to bf16 / fp32 cut into three planes
@@ -37,7 +33,8 @@ template <int XM, int TM>
 struct ShortTile {
   static_assert(TM == 128 || TM == 64 || TM == 32, "row tiles of 128, 64 or 32 rows");
   static constexpr bool split = XM == kXSplit;
-  static constexpr int threads = split ? 1024 : 512, waves = threads / 64;
+  // split: 1024 threads decode a step faster than 512; 128 rows need 128 registers a thread for their sums alone
+  static constexpr int threads = split && TM < 128 ? 1024 : 512, waves = threads / 64;
   static constexpr int ct = kCells * 4 / threads;            // columns of a cell that one thread decodes
   static constexpr int planes = split ? 3 : 1;
   static constexpr int bufs = split ? 1 : 2;                 // LDS buffers of a step's tiles
@@ -211,6 +208,21 @@ __device__ __forceinline__ void gemm_short_block(const mtc_tile_desc& d, const i
   uint32_t w[R], sc[R][SW], base[R];
   u32x4_t q[R][NQ];
   const int cell = tid / (4 / NC), cpart = tid % (4 / NC);   // columns cpart * NC .. of the cell
+  // a gathered cell's scale words: with the descriptor, or with the payload where a whole cell's would take the
+  // registers of a second slot (128-row tiles of fp32 results)
+  constexpr bool kLateScales = PC && T::split && NC == 4;
+  auto load_col_scales = [&](int i, int s) __attribute__((always_inline)) {
+    const uint32_t so = (uint32_t)((i * kCells + cell) * cw) * 4u + 4u + (gcols ? 4u * NC * cpart : 0u);
+    if constexpr (NC == 2) {
+      const u32x2_t v = __builtin_amdgcn_raw_buffer_load_b64(cell_r, so, 0, 0);
+      sc[s][0] = v.x;
+      sc[s][1] = v.y;
+    } else {
+      const u32x4_t v = __builtin_amdgcn_raw_buffer_load_b128(cell_r, so, 0, 0);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) sc[s][SW == 4 ? j : 0] = v[j];
+    }
+  };
   auto load_desc = [&](int i, int s) __attribute__((always_inline)) {
     const uint32_t off = (uint32_t)((i * kCells + cell) * cw) * 4u;
     if constexpr (kCF == kCellBf16) {
@@ -224,16 +236,7 @@ __device__ __forceinline__ void gemm_short_block(const mtc_tile_desc& d, const i
       sc[s][1] = v.z;
     } else {
       w[s] = __builtin_amdgcn_raw_buffer_load_b32(cell_r, off, 0, 0);
-      const uint32_t so = off + 4u + (gcols ? 4u * NC * cpart : 0u);
-      if constexpr (NC == 2) {
-        const u32x2_t v = __builtin_amdgcn_raw_buffer_load_b64(cell_r, so, 0, 0);
-        sc[s][0] = v.x;
-        sc[s][1] = v.y;
-      } else {
-        const u32x4_t v = __builtin_amdgcn_raw_buffer_load_b128(cell_r, so, 0, 0);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) sc[s][j] = v[j];
-      }
+      if constexpr (!kLateScales) load_col_scales(i, s);
     }
     base[s] = step_off[min(i, nks - 1)];
   };
@@ -241,7 +244,8 @@ __device__ __forceinline__ void gemm_short_block(const mtc_tile_desc& d, const i
   auto payload_at = [&](int s, uint32_t cls) __attribute__((always_inline)) {
     return (base[s] + (w[s] & 0x3FFFu)) * 4u + (uint32_t)cpart * ((4u * NC) << (cls & 3u));
   };
-  auto load_payload = [&](int s) __attribute__((always_inline)) {
+  auto load_payload = [&](int i, int s) __attribute__((always_inline)) {
+    if constexpr (kLateScales) load_col_scales(i, s);
     const uint32_t cls = (w[s] >> 14) & 3u, o = payload_at(s, cls);
     q[s][0] = __builtin_amdgcn_raw_buffer_load_b128(pay_r, cls < 3 ? o : kOutOfRange, 0, 0);
     if constexpr (NQ == 2)
@@ -326,9 +330,9 @@ __device__ __forceinline__ void gemm_short_block(const mtc_tile_desc& d, const i
       }
     }
     const int col = (int)(pos >> 3) * 4 + cpart * NC, seg = (int)(pos & 7u);
-    float o[NC][8];
-    decode_cols_f32<PC, NC>(cls, pw, st, sb, o);
     if constexpr (!T::split) {
+      float o[NC][8];
+      decode_cols_f32<PC, NC>(cls, pw, st, sb, o);
 #pragma unroll
       for (int j = 0; j < NC; ++j)
         *reinterpret_cast<u32x4_t*>(bs + swz(col + j, seg)) = u32x4_t{
@@ -341,22 +345,37 @@ __device__ __forceinline__ void gemm_short_block(const mtc_tile_desc& d, const i
       constexpr bool LO = kCF == kCellFp32;
       if (!LO && wide && lane == 0) flags[i & 3] = 1u;
       wide_pos = !LO && cls == 2 ? pos : kCells;
+      // two columns at a time: all four of a whole cell at once take registers that the sums need
 #pragma unroll
-      for (int j = 0; j < NC; ++j) {
-        u32x4_t p[3];
-        unsigned char* const at = bs + swz(col + j, seg);
-        split_planes<LO, false>(o[j], p[0], p[1], p[2], nf);
-        *reinterpret_cast<u32x4_t*>(at) = p[0];
-        *reinterpret_cast<u32x4_t*>(at + T::b_plane) = p[1];
-        if constexpr (LO) *reinterpret_cast<u32x4_t*>(at + 2 * T::b_plane) = p[2];
-      }
-      if (!LO && wide) {                                     // P16 cells: the third plane (zeros elsewhere)
+      for (int j2 = 0; j2 < NC; j2 += 2) {
+        uint32_t pw2[8];                                     // their dwords: from 1, 2 or 4 times j2 on
 #pragma unroll
-        for (int j = 0; j < NC; ++j) {
-          u32x4_t p[3];
-          split_planes<true, false>(o[j], p[0], p[1], p[2], nf);
-          if (cls == 2) *reinterpret_cast<u32x4_t*>(bs + 2 * T::b_plane + swz(col + j, seg)) = p[2];
+        for (int e = 0; e < 8; ++e) {
+          pw2[e] = pw[4 * j2 + e];
+          if (j2 > 0 && e < 4) pw2[e] = cls == 1 ? pw[2 * j2 + e] : pw2[e];
+          if (j2 > 0 && e < 2) pw2[e] = cls == 0 ? pw[j2 + e] : pw2[e];
         }
+        const float st2[2] = {st[j2], st[j2 + 1]}, sb2[2] = {sb[j2], sb[j2 + 1]};
+        float o[2][8];
+        decode_cols_f32<PC, 2>(cls, pw2, st2, sb2, o);
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          u32x4_t p[3];
+          unsigned char* const at = bs + swz(col + j2 + j, seg);
+          split_planes<LO, false>(o[j], p[0], p[1], p[2], nf);
+          *reinterpret_cast<u32x4_t*>(at) = p[0];
+          *reinterpret_cast<u32x4_t*>(at + T::b_plane) = p[1];
+          if constexpr (LO) *reinterpret_cast<u32x4_t*>(at + 2 * T::b_plane) = p[2];
+        }
+        if (!LO && wide) {                                   // P16 cells: the third plane (zeros elsewhere)
+#pragma unroll
+          for (int j = 0; j < 2; ++j) {
+            u32x4_t p[3];
+            split_planes<true, false>(o[j], p[0], p[1], p[2], nf);
+            if (cls == 2) *reinterpret_cast<u32x4_t*>(bs + 2 * T::b_plane + swz(col + j2 + j, seg)) = p[2];
+          }
+        }
+        if constexpr (NC > 2) __builtin_amdgcn_sched_barrier(0);
       }
     }
   };
@@ -367,54 +386,68 @@ __device__ __forceinline__ void gemm_short_block(const mtc_tile_desc& d, const i
   for (int i = 0; i < T::ri; ++i)
 #pragma unroll
     for (int j = 0; j < T::nj; ++j) acc[i][j] = f32x16_t{};
+  f32x16_t low[T::split ? T::ri : 1][T::split ? T::nj : 1];
+  if constexpr (T::split) {
+#pragma unroll
+    for (int i = 0; i < T::ri; ++i)
+#pragma unroll
+      for (int j = 0; j < T::nj; ++j) low[i][j] = f32x16_t{};
+  }
+  // (low: the sums of all plane pairs but the first)
   const int arow = wm * 32 * T::ri + (lane & 31), bcol = wn * 32 * T::nj + (lane & 31);
-  auto a_frag = [&](const unsigned char* as, int z, int i, int seg) __attribute__((always_inline)) {
-    return *reinterpret_cast<const bf16x8_t*>(as + z * T::a_plane + swz(arow + i * 32, seg));
-  };
-  auto b_frag = [&](const unsigned char* bs, int z, int j, int seg) __attribute__((always_inline)) {
-    return *reinterpret_cast<const bf16x8_t*>(bs + z * T::b_plane + swz(bcol + j * 32, seg));
+  // Operand addresses within a plane: 16-row slice kk of the step flips bits 1 and 2 of the segment, 32 more rows are
+  // 4 KiB on (swz). Formed for each slice from one register a tile: kept for all slices they cost spills.
+  constexpr int KK = kTK / 16 / T::wk;                       // 16-row slices of this wave
+  const uint32_t a_at0 = swz(arow, wk * KK * 2 + (lane >> 5)), b_at0 = swz(bcol, wk * KK * 2 + (lane >> 5));
+  auto frag = [&](const unsigned char* plane, uint32_t at, int t) __attribute__((always_inline)) {
+    return *reinterpret_cast<const bf16x8_t*>(plane + at + t * 32 * 128);
   };
   auto mfma_step = [&](const unsigned char* as, const unsigned char* bs, bool third) __attribute__((always_inline)) {
-    constexpr int KK = kTK / 16 / T::wk;                     // 16-row slices of this wave
+    uint32_t a_at = a_at0, b_at = b_at0;
+    if constexpr (T::split) asm volatile("" : "+v"(a_at), "+v"(b_at));
 #pragma unroll
     for (int kk = 0; kk < KK; ++kk) {
-      const int seg = (wk * KK + kk) * 2 + (lane >> 5);
+      const uint32_t ao = a_at ^ (uint32_t)(kk << 5), bo = b_at ^ (uint32_t)(kk << 5);
       bf16x8_t a[NP][T::ri], b[T::split ? 2 : 1][T::nj];
 #pragma unroll
-      for (int z = 0; z < NP; ++z) {
+      for (int z = 0; z < (T::split ? 2 : 1); ++z)
 #pragma unroll
-        for (int i = 0; i < T::ri; ++i) a[z][i] = a_frag(as, z, i, seg);
-        if (z < 2) {
+        for (int j = 0; j < T::nj; ++j) b[z][j] = frag(bs + z * T::b_plane, bo, j);
 #pragma unroll
-          for (int j = 0; j < T::nj; ++j) b[z][j] = b_frag(bs, z, j, seg);
+      for (int i = 0; i < T::ri; ++i) {
+#pragma unroll
+        for (int z = 0; z < NP; ++z) a[z][i] = frag(as + z * T::a_plane, ao, i);
+        auto products = [&](f32x16_t (&c)[T::ri][T::nj], int zb, int za) __attribute__((always_inline)) {
+#pragma unroll
+          for (int j = 0; j < T::nj; ++j)
+            c[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[za][i], b[zb][j], c[i][j], 0, 0, 0);
+        };
+        if constexpr (T::split) {
+          products(acc, 0, 0);
+          products(low, 1, 1);
+          products(low, 0, 2);
+          products(low, 1, 0);
+          products(low, 0, 1);
+          __builtin_amdgcn_sched_barrier(0);                 // one slice's operands in registers at a time
+        } else {
+          products(acc, 0, 0);
         }
       }
-      auto products = [&](int zb, int za) __attribute__((always_inline)) {
-#pragma unroll
-        for (int i = 0; i < T::ri; ++i)
-#pragma unroll
-          for (int j = 0; j < T::nj; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[za][i], b[zb][j], acc[i][j], 0, 0, 0);
-      };
-      if constexpr (T::split) {
-        products(1, 1);
-        products(0, 2);
-        products(1, 0);
-        products(0, 1);
-      }
-      products(0, 0);
-      if constexpr (T::split) __builtin_amdgcn_sched_barrier(0);   // one slice's operands in registers at a time
     }
-    if (T::split && third) {                                 // the weights' third plane . X's first
+    if constexpr (T::split) if (third) {                     // the weights' third plane . X's first
 #pragma unroll
       for (int kk = 0; kk < KK; ++kk) {
-        const int seg = (wk * KK + kk) * 2 + (lane >> 5);
+        const uint32_t ao = a_at ^ (uint32_t)(kk << 5), bo = b_at ^ (uint32_t)(kk << 5);
 #pragma unroll
-        for (int i = 0; i < T::ri; ++i)
+        for (int i = 0; i < T::ri; ++i) {
+          const bf16x8_t a0 = frag(as, ao, i);
 #pragma unroll
-          for (int j = 0; j < T::nj; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a_frag(as, 0, i, seg), b_frag(bs, 2, j, seg), acc[i][j],
-                                                                0, 0, 0);
+          for (int j = 0; j < T::nj; ++j) {
+            const bf16x8_t b2 = frag(bs + 2 * T::b_plane, bo, j);
+            low[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a0, b2, low[i][j], 0, 0, 0);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
       }
     }
   };
@@ -423,11 +456,15 @@ __device__ __forceinline__ void gemm_short_block(const mtc_tile_desc& d, const i
   auto step = [&](int i, int s, XRegs& x) __attribute__((always_inline)) {
     unsigned char* const as = lds + (T::bufs == 2 ? (i & 1) * T::buf_bytes : 0);
     unsigned char* const bs = as + NP * T::a_plane;
+    if constexpr (T::split && TM == 128) {                   // X first: the decode then takes its registers
+      store_x(as, x);
+      __builtin_amdgcn_sched_barrier(0);
+    }
     stage_cell(bs, s, i);
-    store_x(as, x);
+    if constexpr (!(T::split && TM == 128)) store_x(as, x);
     load_x(i + T::xring, x);                                 // first: loads return in order, and the next step waits for X
     load_desc(i + R, s);
-    load_payload((s + R - 1) % R);
+    load_payload(i + R - 1, (s + R - 1) % R);
     bool third = kCF == kCellFp32;
     if constexpr (T::split && kCF != kCellFp32) {
       if (tid == 0) flags[(i + 2) & 3] = 0u;
@@ -446,22 +483,22 @@ __device__ __forceinline__ void gemm_short_block(const mtc_tile_desc& d, const i
       lds_barrier();
     }
   };
-  if (T::split) {
-    if (tid < 5) flags[tid] = 0u;
-    unsigned char* const third_plane = lds + NP * T::a_plane + 2 * T::b_plane;
-#pragma unroll
-    for (int z = 0; z < T::b_plane / (16 * T::threads); ++z)
-      *reinterpret_cast<u32x4_t*>(third_plane + (z * T::threads + tid) * 16) = u32x4_t{0u, 0u, 0u, 0u};
-    lds_barrier();
-  }
   // the first step's payload ahead of the later steps' descriptors, which would queue in front of it
   load_desc(0, 0);
   load_x(0, xr[0]);
 #pragma unroll
   for (int s = 1; s < R; ++s) {
     load_desc(s, s);
-    load_payload(s - 1);
+    load_payload(s - 1, s - 1);
     if (s == 1 && T::xring == 2) load_x(1, xr[T::xring - 1]);
+  }
+  if (T::split) {                                            // (while the first loads are in flight)
+    if (tid < 5) flags[tid] = 0u;
+    unsigned char* const third_plane = lds + NP * T::a_plane + 2 * T::b_plane;
+#pragma unroll
+    for (int z = 0; z < T::b_plane / (16 * T::threads); ++z)
+      *reinterpret_cast<u32x4_t*>(third_plane + (z * T::threads + tid) * 16) = u32x4_t{0u, 0u, 0u, 0u};
+    lds_barrier();
   }
   static_assert(R % T::xring == 0, "the X registers' ring divides the cells'");
   for (int i0 = 0; i0 < nks; i0 += R) {
@@ -475,6 +512,12 @@ __device__ __forceinline__ void gemm_short_block(const mtc_tile_desc& d, const i
   const int64_t ld = part ? (int64_t)d.N : ldy;
   const bool fp32_out = part || kYDT == MTC_DTYPE_F32;
   if constexpr (T::split) {
+#pragma unroll
+    for (int i = 0; i < T::ri; ++i)
+#pragma unroll
+      for (int j = 0; j < T::nj; ++j)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[i][j][e] += low[i][j][e];
     if (nf != nf) flags[4] = 1u;
     __syncthreads();
     if (flags[4]) {

@@ -7,7 +7,7 @@ import pytest
 from oracle import mtc_oracle as O
 from tensorpack_amd.core.allocation import rd_allocate
 from tensorpack_amd.core.permutation import PermutedQuadtreeRD
-from tensorpack_amd.core.quadtree import QuadtreeRD
+from tensorpack_amd.core.quadtree import QTAllocation, QuadtreeRD
 from tensorpack_amd.kernels.gemm import MTCMatrix
 
 from conftest import outlier_matrix
@@ -92,3 +92,35 @@ def test_f32_tiles_infinities_nan_and_range(gpu, mats, form, M):
     Yt = t.gemm_f32(torch.from_numpy(tiny).to(gpu)).cpu().numpy().astype(np.float64)
     ref = tiny.astype(np.float64) @ W_hat.astype(np.float64)
     assert np.abs(Yt - ref).max() <= K * 2.0 ** -126 * np.abs(W_hat).max()
+
+
+def _flat(W, P, scales, S=32):
+    """A matrix of S x S leaves of one code width, with the given bf16 scales, and its W_hat."""
+    K, N = W.shape
+    leaf, modes = {S: np.ones((K // S, N // S), bool)}, {S: np.full((K // S, N // S), P)}
+    a = QTAllocation((S,), leaf, modes, {S: scales}, None, K * N * P, weights=W)
+    return MTCMatrix.from_quadtree(a), O.qt_dequant(W, (S,), leaf, modes, {S: scales})
+
+
+@pytest.mark.parametrize("form", ["qt", "p16", "uniform"])
+def test_f32_same_signed_sums(gpu, form):
+    """Sums of one sign over 8192 rows that are not split: two, two or three and three weight planes. The
+    small plane products must not fall below half an ulp of the running sum, which loses them all to one side."""
+    import torch
+    K, N, M = 8192, 2048, 4096
+    rng = np.random.RandomState(5)
+    W = (0.5 + rng.rand(K, N)).astype(np.float32)
+    if form == "uniform":
+        s = np.exp(-4.4 + 0.1 * rng.rand(K // 32, N // 32)).astype(np.float32)
+        m = MTCMatrix.from_allocation(W, np.full((K // 32, N // 32), 8, np.uint8), s, 32)
+        W_hat = O.uniform_to_array(W, np.full((K // 32, N // 32), 8, np.uint8), s, 32)
+    else:
+        m, W_hat = _flat(W, 16 if form == "p16" else 8, np.full((K // 32, N // 32), 2.0 ** (-14 if form == "p16" else -6), np.float32))
+    t = m.device_tiles(gpu)
+    X = torch.from_numpy((0.5 + rng.rand(M, K)).astype(np.float32)).to(gpu)
+    print("f32 same-signed", form, flush=True)
+    Y = t.gemm_f32(X).double()
+    ref = X.double() @ torch.from_numpy(W_hat).to(gpu).double()
+    # rounded once per 16 rows of K (one MFMA), each time by up to half an ulp of the running sum: a random walk
+    assert ((Y - ref).norm() / ref.norm()).item() <= (np.sqrt(K / 16) + 2) * 2.0 ** -24
+    assert abs(((Y - ref).mean() / ref.mean()).item()) <= 2.0 ** -24       # to neither side
