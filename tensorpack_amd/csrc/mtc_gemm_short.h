@@ -16,13 +16,16 @@
 // each the upper half of what the planes before left (8 + 8 + 8 significant bits: exact, mid below 2^-7 and
 // lo below 2^-15 of hi's leading bit). X takes three planes; a weight code * scale with a code of at most
 // 8 bits and a bf16 scale has at most 16 significant bits and takes two, a P16 code or an fp32 scale three.
-// Products of bf16 values are exact in fp32; all pairs of planes are multiplied but (weight . X) mid.lo, lo.mid
-// and lo.lo. v_mfma_f32_32x32x16_bf16 does 16 times the products
-// per clock of v_mfma_f32_16x16x4f32, for five or six times the number.
+// Products of bf16 values are exact in fp32, and every pair of planes is multiplied but lo.lo of
+// three-plane weights (below 2^-30 of the product). v_mfma_f32_32x32x16_bf16 does 16 times the products
+// per clock of v_mfma_f32_16x16x4f32, for six or eight times the number.
 //   Two accumulators: hi.hi in one, the other pairs in a second that is added at the end. In one, the small
 // pairs of a slice fall below half an ulp of a long sum of one sign, always to the same side.
 //   X or weights that are not finite have no planes (inf - inf): a block that met one computes its tile again
 // in plain fp32.
+// Error against fp64, 2-norm, 4096 x 4096 QT @ 4.5 (an fma chain in K order: the fp32 MFMAs of 16-row tiles):
+// M = 100 1.2e-7 (6.0e-7), M = 2048 3.4e-7 (1.0e-6); X and W positive, M = 2048 3.0e-7 (8.6e-7), 8192 x 4096
+// 4.3e-7 (1.2e-6); one product alone 2.5e-8 (2.5e-8).
 #pragma once
 
 enum { kXBf16, kXRound, kXSplit };   // X: bf16 / fp32 rounded to bf16 / fp32 cut into three planes
@@ -423,6 +426,7 @@ __device__ __forceinline__ void gemm_short_block(const mtc_tile_desc& d, const i
             c[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[za][i], b[zb][j], c[i][j], 0, 0, 0);
         };
         if constexpr (T::split) {
+          products(low, 1, 2);
           products(acc, 0, 0);
           products(low, 1, 1);
           products(low, 0, 2);
@@ -434,16 +438,17 @@ __device__ __forceinline__ void gemm_short_block(const mtc_tile_desc& d, const i
         }
       }
     }
-    if constexpr (T::split) if (third) {                     // the weights' third plane . X's first
+    if constexpr (T::split) if (third) {                     // the weights' third plane . X's first two
 #pragma unroll
       for (int kk = 0; kk < KK; ++kk) {
         const uint32_t ao = a_at ^ (uint32_t)(kk << 5), bo = b_at ^ (uint32_t)(kk << 5);
 #pragma unroll
         for (int i = 0; i < T::ri; ++i) {
-          const bf16x8_t a0 = frag(as, ao, i);
+          const bf16x8_t a1 = frag(as + T::a_plane, ao, i), a0 = frag(as, ao, i);
 #pragma unroll
           for (int j = 0; j < T::nj; ++j) {
             const bf16x8_t b2 = frag(bs + 2 * T::b_plane, bo, j);
+            low[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a1, b2, low[i][j], 0, 0, 0);
             low[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a0, b2, low[i][j], 0, 0, 0);
           }
           __builtin_amdgcn_sched_barrier(0);

@@ -124,3 +124,34 @@ def test_f32_same_signed_sums(gpu, form):
     # rounded once per 16 rows of K (one MFMA), each time by up to half an ulp of the running sum: a random walk
     assert ((Y - ref).norm() / ref.norm()).item() <= (np.sqrt(K / 16) + 2) * 2.0 ** -24
     assert abs(((Y - ref).mean() / ref.mean()).item()) <= 2.0 ** -24       # to neither side
+
+
+@pytest.mark.parametrize("form", ["qt", "p16", "uniform"])
+def test_f32_single_products(gpu, form):
+    """One non-zero X a row: every output is one product, right to its own rounding and the sum of the small
+    plane products' (some are left out below 2^-30). Mantissas whose middle and low planes are as large as
+    they get."""
+    import torch
+    K = N = 256
+    if form == "qt":                       # 79 * 209 = 0x407F: two planes, the second 0xFE
+        W = np.full((K, N), 79 * 209 * 2.0 ** -14, np.float32)
+        m, W_hat = _flat(W, 8, np.full((8, 8), 209 * 2.0 ** -14, np.float32))
+    elif form == "p16":                    # 20382 * 209 = 0x40FFFE: three planes
+        W = np.full((K, N), 20382 * 209 * 2.0 ** -22, np.float32)
+        m, W_hat = _flat(W, 16, np.full((8, 8), 209 * 2.0 ** -22, np.float32))
+    else:
+        s = np.full((8, 8), np.float32(0x80FFFF * 2.0 ** -23) / np.float32(127), np.float32)
+        W = np.full((K, N), np.float32(127) * s[0, 0], np.float32)
+        m = MTCMatrix.from_allocation(W, np.full((8, 8), 8, np.uint8), s, 32)
+        W_hat = O.uniform_to_array(W, np.full((8, 8), 8, np.uint8), s, 32)
+    low = W_hat.view(np.uint32) & 0xFFFF
+    assert (low >= 0xFE00).all()                                           # the planes the test is about
+    t = m.device_tiles(gpu)
+    for M in (20, 64, 200):
+        X = np.zeros((M, K), np.float32)
+        X[np.arange(M), np.arange(M) % K] = np.array([0x3F80FFFF, 0xBFFFFFFF], np.uint32).view(np.float32)[np.arange(M) % 2]
+        print("f32 single products", form, M, flush=True)
+        Y = t.gemm_f32(torch.from_numpy(X).to(gpu)).cpu().numpy()
+        ref = X.astype(np.float64) @ W_hat.astype(np.float64)
+        # half an ulp of the result, and half an ulp of each of the sums of the small pairs: they are below 2^-6 of it
+        assert (np.abs(Y - ref) <= np.abs(ref) * (2.0 ** -24 + 8 * 2.0 ** -30)).all(), np.abs(Y / ref - 1).max()
