@@ -321,11 +321,12 @@ int mtc_set_prefill_decode_once(int enable);
 
 /* fp32 matrix-core path over the tile stream: Y (M x N fp32, leading dim ldy) = X (M x K
  * fp32, leading dim ldx) * W_hat with the exact fp32 W_hat, fp32 X and fp32 sums: both are cut into
- * bf16 planes whose products are exact in fp32 (v_mfma_f32_32x32x16_bf16 over plane pairs; pairs below
- * 2^-24 of the product are left out), in tiles of 32, 64 or 128 rows with K split over blocks until the
- * chip is full; within the fp32 tolerance of the reference's float32 block loop
- * (mtc/kernels/gemm.py:124-210, the same operation as mtc_gemv_f32, for callers at 5..16 rows and
- * beyond). Values that are not finite give what a plain fp32 loop gives. X read in place
+ * bf16 planes whose products are exact in fp32 (v_mfma_f32_32x32x16_bf16 over the plane pairs; only the
+ * pair of two third planes, below 2^-30 of the product, is left out), in tiles of 32, 64 or 128 rows with
+ * K split over blocks until the chip is full; within the fp32 tolerance of the reference's float32 block
+ * loop (mtc/kernels/gemm.py:124-210, the same operation as mtc_gemv_f32, for callers at 5..16 rows and
+ * beyond), subnormal values included. Values that are not finite or from 2^104 on, and sums from 2^80 on,
+ * give what a plain fp32 loop gives, at its speed: the tiles that meet them run it. X read in place
  * must have 16-byte aligned rows (ldx % 4 == 0); a stream with a row permutation gathers X
  * into the workspace first. Workspace (mtc_gemm_f32_workspace_bytes, 256-byte aligned, no
  * initialisation): the gathered X (M*K*4) and the split-K partials.

@@ -21,16 +21,19 @@
 // per clock of v_mfma_f32_16x16x4f32, for six or eight times the number.
 //   Two accumulators: hi.hi in one, the other pairs in a second that is added at the end. In one, the small
 // pairs of a slice fall below half an ulp of a long sum of one sign, always to the same side.
-//   X or weights that are not finite have no planes (inf - inf): a block that met one computes its tile again
-// in plain fp32.
+//   X and the scales are multiplied by 2^24 first and the sums by 2^-48 at the end: then every bit of an
+// fp32 value, of a subnormal one too, is a normal bf16 number, where the low planes of values under 2^-109
+// would lose bits below 2^-133. X or weights that are not finite have no planes (inf - inf), and values from
+// 2^104 or sums from 2^80 on overflow: a block that met one computes its tile again in plain fp32.
 // Error against fp64, 2-norm, 4096 x 4096 QT @ 4.5 (an fma chain in K order: the fp32 MFMAs of 16-row tiles):
 // M = 100 1.2e-7 (6.0e-7), M = 2048 3.4e-7 (1.0e-6); X and W positive, M = 2048 3.0e-7 (8.6e-7), 8192 x 4096
-// 4.3e-7 (1.2e-6); one product alone 2.5e-8 (2.5e-8).
+// 4.3e-7 (1.2e-6); X times 2^-124 1.2e-7 (6.1e-7); one product alone 2.5e-8 (2.5e-8).
 #pragma once
 
 enum { kXBf16, kXRound, kXSplit };   // X: bf16 / fp32 rounded to bf16 / fp32 cut into three planes
 
 constexpr int kShortFlagBytes = 64;
+constexpr float kPlaneScale = 0x1p24f;   // of X and the scales ahead of the planes (see above)
 
 template <int XM, int TM>
 struct ShortTile {
@@ -292,6 +295,8 @@ __device__ __forceinline__ void gemm_short_block(const mtc_tile_desc& d, const i
               u32x4_t{pk_bf16(v[0], v[1]), pk_bf16(v[2], v[3]), pk_bf16(v[4], v[5]), pk_bf16(v[6], v[7])};
         } else {
           u32x4_t p[3];
+#pragma unroll
+          for (int e = 0; e < 8; ++e) v[e] *= kPlaneScale;
           split_planes<true, true>(v, p[0], p[1], p[2], nf);
 #pragma unroll
           for (int z = 0; z < 3; ++z) *reinterpret_cast<u32x4_t*>(at + z * T::a_plane) = p[z];
@@ -330,6 +335,13 @@ __device__ __forceinline__ void gemm_short_block(const mtc_tile_desc& d, const i
         const uint32_t v = gcols ? own : first;
         st[j] = __uint_as_float(v << 16);
         sb[j] = __uint_as_float(v & 0xFFFF0000u);
+      }
+    }
+    if constexpr (T::split) {
+#pragma unroll
+      for (int j = 0; j < NC; ++j) {
+        st[j] *= kPlaneScale;
+        sb[j] *= kPlaneScale;
       }
     }
     const int col = (int)(pos >> 3) * 4 + cpart * NC, seg = (int)(pos & 7u);
@@ -522,7 +534,11 @@ __device__ __forceinline__ void gemm_short_block(const mtc_tile_desc& d, const i
 #pragma unroll
       for (int j = 0; j < T::nj; ++j)
 #pragma unroll
-        for (int e = 0; e < 16; ++e) acc[i][j][e] += low[i][j][e];
+        for (int e = 0; e < 16; ++e) {
+          acc[i][j][e] += low[i][j][e];
+          nf = __builtin_fmaf(acc[i][j][e], 0.0f, nf);
+          acc[i][j][e] *= 1.0f / (kPlaneScale * kPlaneScale);
+        }
     if (nf != nf) flags[4] = 1u;
     __syncthreads();
     if (flags[4]) {

@@ -155,3 +155,29 @@ def test_f32_single_products(gpu, form):
         ref = X.astype(np.float64) @ W_hat.astype(np.float64)
         # half an ulp of the result, and half an ulp of each of the sums of the small pairs: they are below 2^-6 of it
         assert (np.abs(Y - ref) <= np.abs(ref) * (2.0 ** -24 + 8 * 2.0 ** -30)).all(), np.abs(Y / ref - 1).max()
+
+
+@pytest.mark.parametrize("form", ["qt", "qtp", "p16", "uniform"])
+def test_f32_small_magnitudes(gpu, mats, form):
+    """Normal fp32 inputs whose low bf16 planes would be below bf16's range, and such weights, cost no bits."""
+    import torch
+    m, W_hat = mats["ragged", form]
+    K = W_hat.shape[0]
+    t = m.device_tiles(gpu)
+    for M in (17, 64, 100):
+        X = np.random.RandomState(M).randn(M, K).astype(np.float32)
+        for e in (-100, -112, -116, -120):
+            Xe = (X * 2.0 ** e).astype(np.float32)
+            print("f32 small magnitudes", form, M, e, flush=True)
+            Y = t.gemm_f32(torch.from_numpy(Xe).to(gpu)).cpu().numpy()
+            up = 2.0 ** -e                     # exact in 64 bits: the error function's floor is far above these values
+            assert O.relative_frobenius_error(O.qt_gemm_f64(Xe, W_hat) * up, Y.astype(np.float64) * up) <= _tol(K), (M, e)
+    if form == "uniform":
+        rng = np.random.RandomState(9)
+        W = (rng.randn(K, 288) * 2.0 ** -112).astype(np.float32)
+        modes = np.full((K // 32, 9), 8, np.uint8)
+        s = (np.exp(0.1 * rng.rand(K // 32, 9)) * 2.0 ** -117).astype(np.float32)
+        w, W_hat = MTCMatrix.from_allocation(W, modes, s, 32).device_tiles(gpu), O.uniform_to_array(W, modes, s, 32)
+        Y = w.gemm_f32(torch.from_numpy(X).to(gpu)).cpu().numpy()
+        up = 2.0 ** 112
+        assert O.relative_frobenius_error(O.qt_gemm_f64(X, W_hat) * up, Y.astype(np.float64) * up) <= _tol(K)
