@@ -339,6 +339,10 @@ size_t mtc_gemm_f32_workspace_bytes(const mtc_tile_desc* d, int M);
 int mtc_gemm_f32(const mtc_tile_desc* d, const float* X, int64_t ldx, float* Y, int64_t ldy, int M,
                  void* workspace, size_t workspace_bytes, void* hip_stream);
 
+/* Rows per output tile and K splits that the tile kernels choose for M rows of X: mtc_gemm_f32's, or
+ * with fp32_results 0 mtc_gemm_bf16's where it does not take the decode-once path. Host only. */
+int mtc_tile_plan(const mtc_tile_desc* d, int M, int fp32_results, int* tile_rows, int* k_splits);
+
 /* Prefill for n (1..MTC_MAX_GROUP) matrices that read the same X, one launch per kernel
  * (X staging, tile GEMM, split-K reduction) instead of one per matrix:
  * Y[i] (M x N_i, leading dim ldy[i]) = X * W_hat_i. Every tile stream must have the same

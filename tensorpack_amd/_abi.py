@@ -20,7 +20,7 @@ EXPORTED = ("mtc_abi_version", "mtc_last_error", "mtc_check_desc", "mtc_dequant"
             "mtc_gemv_workspace_bytes", "mtc_gemv_f32", "mtc_gemv_f32_group", "mtc_check_tile_desc", "mtc_tile_dequant", "mtc_gemm_workspace_bytes",
             "mtc_gemm_bf16", "mtc_gemm_group_workspace_bytes", "mtc_gemm_bf16_group", "mtc_gemv_batch_plan",
             "mtc_gemv_f32_batch", "mtc_gemv_noalloc_scratch_bytes", "mtc_gemv_f32_noalloc", "mtc_gemm_batch_plan",
-            "mtc_gemm_bf16_batch", "mtc_gemm_f32_workspace_bytes", "mtc_gemm_f32",
+            "mtc_gemm_bf16_batch", "mtc_gemm_f32_workspace_bytes", "mtc_gemm_f32", "mtc_tile_plan",
             "mtc_set_prefill_decode_once")
 
 
@@ -135,6 +135,8 @@ def declare(lib: ctypes.CDLL) -> None:
     lib.mtc_check_tile_desc.argtypes = [TileDescP]
     lib.mtc_tile_dequant.restype = i32
     lib.mtc_tile_dequant.argtypes = [TileDescP, vp, vp]
+    lib.mtc_tile_plan.restype = i32
+    lib.mtc_tile_plan.argtypes = [TileDescP, i32, i32, ctypes.POINTER(i32), ctypes.POINTER(i32)]
     lib.mtc_gemm_workspace_bytes.restype = sz
     lib.mtc_gemm_workspace_bytes.argtypes = [TileDescP, i32, i32]
     lib.mtc_gemm_bf16.restype = i32

@@ -1831,39 +1831,43 @@ MTC_API int mtc_gemm_bf16_batch(const void* host_plan, const void* device_plan, 
 MTC_API int mtc_check_tile_desc(const mtc_tile_desc* d) { return check_tile_desc(d); }
 
 // ---- fp32 tile path (k_gemm_f32) ----
-// Tile height and K split of an fp32 call: the height (32, 64 or 128 rows) and split count (at most
-// enough blocks to fill the chip, at least kMinStepsPerSplit K-steps each) with the least estimated time, as
-// tile_plan estimates it.
+// Tile height and K split of an fp32 call: the height (32, 64 or 128 rows) and split count (at most two
+// rounds of blocks) with the least estimated time, estimated as tile_plan does: rounds of blocks on the
+// fullest XCD, the K-steps of a block, and the split-K partials.
 struct F32Plan {
   int tm;        // output rows per tile block
   int splits;
   int per;       // K-steps per split
 };
-// Time of one K-step of an fp32 block by its row-tile height (one block alone over 128 steps): decode
-// 1.2-1.4 us, then the MFMAs, 0.5 us for 32 rows, 1.1 for 64 and 2.2 (their peak rate) for 128. kF32BlockUs:
-// launch to the first step's data; the partials move faster than the bf16 path's (4096 x 4096, M = 100 with
-// 16 splits of 128 rows 39.1 us, 8 of 64 rows 39.2, 4 of 32 rows 45.3; M = 256 59.8, 62.0, 76.4).
-constexpr double kF32BlockUs = 7.0;
-constexpr double kF32ReduceBytesPerUs = 5.0e6;
-inline double f32_step_us(int tm) { return tm == 128 ? 3.6 : tm == 64 ? 2.4 : 1.75; }
-F32Plan f32_plan(const mtc_tile_desc* d, int M, int64_t ldx = 0) {
-  const double split_bytes = 2.0 * 4.0 * (double)M * d->N;     // one partial, written and read
+// Time of one K-step of a block by its height, of its launch to the first step's data (kF32BlockUs) and of
+// the partials' traffic, fitted to shapes timed with forced plans (profiles/f32_tile_plans.txt). Counted on
+// the whole chip, 3 splits of 85 tiles fit one round of 256 blocks but are 33 on an XCD's 32 CUs:
+// 1664 x 4224 QT, M = 545, 95.6 us (64 rows x 3 splits, 459 blocks: 69.3); 2464 x 2816, M = 155, 43.4
+// against 31.4. A split may be a single K-step: 20 x 256 x 256 9.7 us in 4 splits of one, 11.7 in 2 of two.
+constexpr double kF32BlockUs = 3.6;
+constexpr double kF32ReduceBytesPerUs = 6.0e6;
+inline double f32_step_us(int tm) { return tm == 128 ? 5.0 : tm == 64 ? 2.9 : 1.9; }
+// max_tm, max_splits: bounds for a call whose X rows are too far apart for a taller block's 32-bit offsets.
+F32Plan f32_plan(const mtc_tile_desc* d, int M, int max_tm = 128, int max_splits = 1 << 30) {
+  const double split_us = 2.0 * 4.0 * (double)M * d->N / kF32ReduceBytesPerUs;   // one partial, written and read
+  constexpr int64_t xcd_cus = kFillCUs / kXcds;
   F32Plan best{0, 1, d->n_ksteps};
   double best_t = 1e300;
   for (int tm : {32, 64, 128}) {
-    if (tm > 32 && (M <= tm / 2 || ldx >= ((int64_t)1 << 30) / tm)) break;   // 32-bit offsets within a block's X rows
+    if (tm > 32 && (M <= tm / 2 || tm > max_tm)) break;
     const int64_t n_tiles = (int64_t)((M + tm - 1) / tm) * d->n_col_tiles;
-    int max_s = n_tiles >= kFillCUs ? 1 : (int)((kFillCUs + n_tiles - 1) / n_tiles);
-    max_s = std::max(1, std::min(max_s, d->n_ksteps / kMinStepsPerSplit));
+    const int64_t xcd_tiles = (n_tiles + kXcds - 1) / kXcds;
+    int max_s = (int)std::max<int64_t>(1, (2 * kFillCUs + n_tiles - 1) / n_tiles);
+    max_s = std::min({max_s, d->n_ksteps, max_splits});
     for (int s = 1; s <= max_s; ++s) {
       const int per = (d->n_ksteps + s - 1) / s;
-      const int s_eff = (d->n_ksteps + per - 1) / per;
-      const double rounds = std::ceil((double)(n_tiles * s_eff) / kFillCUs);
+      if ((d->n_ksteps + per - 1) / per < s) continue;         // the same plan as fewer splits
+      const double rounds = (double)((xcd_tiles * s + xcd_cus - 1) / xcd_cus);
       const double t = rounds * (per * f32_step_us(tm) + kF32BlockUs) +
-                       (s_eff > 1 ? s_eff * split_bytes / kF32ReduceBytesPerUs + kReduceLaunchUs : 0.0);
+                       (s > 1 ? s * split_us + kReduceLaunchUs : 0.0);
       if (t < best_t) {
         best_t = t;
-        best = {tm, s_eff, per};
+        best = {tm, s, per};
       }
     }
   }
@@ -1912,6 +1916,23 @@ MTC_API size_t mtc_gemm_f32_workspace_bytes(const mtc_tile_desc* d, int M) {
   if (check_tile_desc(d) || M <= 0) return 0;
   const size_t tiles = f32_ws_bytes(d, M);
   return decode_once_f32_shape(d, M) ? std::max(tiles, decode_once_f32_bytes(d, M)) : tiles;
+}
+
+MTC_API int mtc_tile_plan(const mtc_tile_desc* d, int M, int fp32_results, int* tile_rows, int* k_splits) {
+  int rc = check_tile_desc(d);
+  if (rc) return rc;
+  if (!tile_rows || !k_splits) return fail(MTC_E_NULL, "tile_rows or k_splits is NULL");
+  if (M <= 0) return fail(MTC_E_SHAPE, "M=%d must be positive", M);
+  if (fp32_results) {
+    const F32Plan p = f32_plan(d, M);
+    *tile_rows = p.tm;
+    *k_splits = p.splits;
+  } else {
+    const TilePlan p = tile_plan(d, M);
+    *tile_rows = p.tm;
+    *k_splits = p.splits;
+  }
+  return ok();
 }
 
 MTC_API int mtc_gemm_f32(const mtc_tile_desc* d, const float* X, int64_t ldx, float* Y, int64_t ldy, int M,
@@ -1978,7 +1999,9 @@ MTC_API int mtc_gemm_f32(const mtc_tile_desc* d, const float* X, int64_t ldx, fl
     xa = xp;
     lda = d->K;
   }
-  const F32Plan p = f32_plan(d, M, lda);   // a longer row only lowers the tile height, and with it the splits
+  F32Plan p = f32_plan(d, M);
+  if (lda >= ((int64_t)1 << 30) / p.tm)      // a block's X rows span 4 GiB: a lower tile, in the workspace of this plan
+    p = f32_plan(d, M, lda >= (int64_t)1 << 24 ? 32 : 64, p.splits);
   float* part = p.splits > 1 ? reinterpret_cast<float*>(reinterpret_cast<char*>(workspace) + stage) : nullptr;
   switch (cell_format(d)) {
     case kCellFp32: rc = launch_f32<kCellFp32>(d, p, xa, lda, Y, ldy, M, part, st); break;
