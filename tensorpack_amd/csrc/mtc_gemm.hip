@@ -100,14 +100,6 @@ __device__ __forceinline__ uint32_t swz(int row, int seg) {
   return (uint32_t)(row * 128 + ((seg ^ (row & 7) ^ ((row >> 3) & 1)) << 4));
 }
 
-// fp32 tiles of the decode-once path: [rows][64] floats, 256 bytes (all 64 banks) per row, 16-byte
-// segment `seg` (0..15) of row `row` stored at segment seg ^ f(row), f(row) = (row & 15) ^ bit 2 of
-// row, so that the stores of one column of two neighbouring cells (rows n and n + 4, whose f differ in
-// bit 0, at the 8 even or the 8 odd segments) land in different segments.
-__device__ __forceinline__ uint32_t swz_f32(int row, int seg) {
-  return (uint32_t)(row * 256 + ((seg ^ (row & 15) ^ ((row >> 2) & 1)) << 4));
-}
-
 // Hides a value's known bits so byte extraction compiles to v_cvt_f32_ubyteN.
 __device__ __forceinline__ uint32_t opaque(uint32_t x) {
   asm("" : "+v"(x));
@@ -589,20 +581,18 @@ __global__ __launch_bounds__(kStageThreads) void k_stage_x_f32(const float* __re
   *reinterpret_cast<float4*>(Xp + m * K + k0) = make_float4(x[src.x], x[src.y], x[src.z], x[src.w]);
 }
 
-// ---- decode once: W_hat in bf16 (or fp32) for a plain GEMM ----
+// ---- decode once: W_hat in bf16 for a plain GEMM ----
 // One block per (column tile ct, run of `spb` K-steps), grid n_col_tiles x ceil(n_ksteps / spb),
 // 256 threads: for each step thread t decodes cells t and t + 256 as the tile kernel's producers
-// do (decode_cell: the same bf16 values the MFMAs would read; with F32, decode_cell_f32: the exact
-// W_hat) into a swizzled [256][64] LDS tile, then the block writes it out as whole row pieces
-// (128 bytes of bf16, 256 of fp32): Wt[n][k] (N rows of ldw elements, ldw = 64 * n_ksteps) holds
-// W_hat[k][n] for stream row k (row_perm order, as the staged X) and column n; rows k >= K hold
+// do (decode_cell: the same bf16 values the MFMAs would read) into a swizzled [256][64] LDS tile,
+// then the block writes it out as whole row pieces (128 bytes): Wt[n][k] (N rows of ldw elements,
+// ldw = 64 * n_ksteps) holds W_hat[k][n] for stream row k (row_perm order, as the staged X) and column n; rows k >= K hold
 // the stream's zero padding. While a step is decoded and written, the next step's payload and
 // the descriptors of the step after it are in flight. (Stores straight from registers, one cell
 // per thread, ran 54 us against 40 us for one step per block at 8192 x 8192 in bf16: a step's
 // cells are sorted by class first, so their lines split.)
-enum { kOutWtBf16, kOutWtF32, kOutRows };   // what tile_dequant_block writes (kOutRows: see below)
-
-// kOutRows: W_hat itself, fp32, row-major in the original channel order (W: K rows of ldw floats).
+//
+// kRows: W_hat itself, fp32, row-major in the original channel order (W: K rows of ldw floats).
 // Bound by HBM: 4096 x 4096 QT-P @ 4.25 reads 27 MB and writes 67 MB in 17.9 us, 5.2 TB/s (a 1 GiB
 // copy reaches 5.0; the panel stream's k_dequant and its zero fill took 280 us, its 4-byte stores
 // scattered through col_perm). The
@@ -614,11 +604,10 @@ __device__ __forceinline__ uint32_t swz_rows(int row, int seg) {
   return (uint32_t)(row * (kTN * 4) + ((seg ^ ((row >> 3) << 1)) << 4));
 }
 
-template <int kCF, int OUT>
+template <int kCF, bool kRows>
 __device__ __forceinline__ void tile_dequant_block(const mtc_tile_desc& d, void* __restrict__ Wt, int64_t ldw,
                                                    int spb) {
-  constexpr bool F32 = OUT != kOutWtBf16;
-  __shared__ __attribute__((aligned(16))) unsigned char bs[kTN * kTK * (F32 ? 4 : 2)];
+  __shared__ __attribute__((aligned(16))) unsigned char bs[kTN * kTK * (kRows ? 4 : 2)];
   constexpr int CW = cell_words(kCF);
   const int t = threadIdx.x, ct = blockIdx.x;
   const int ks0 = (int)blockIdx.y * spb, nks = min(spb, d.n_ksteps - ks0);
@@ -674,7 +663,7 @@ __device__ __forceinline__ void tile_dequant_block(const mtc_tile_desc& d, void*
       }
       const uint32_t pos = (w[h][0] >> 16) & (kCells - 1);   // (column group, row block) of the cell
       const int col = (int)(pos >> 3) * 4, seg = (int)(pos & 7u);
-      if constexpr (OUT == kOutRows) {
+      if constexpr (kRows) {
         // code times scale, as the panel stream's dequantizer computes it (one rounded product: exact for
         // bf16 scales; no negative zeros in a quadtree W_hat, whose levels are summed into +0.0)
         const float one[4] = {1.0f, 1.0f, 1.0f, 1.0f};
@@ -690,14 +679,6 @@ __device__ __forceinline__ void tile_dequant_block(const mtc_tile_desc& d, void*
           }
           *reinterpret_cast<f32x4_t*>(bs + swz_rows(8 * seg + r, col >> 2)) = v;
         }
-      } else if constexpr (F32) {
-        float o[4][8];
-        decode_cell_f32<kCF == kCellCols>((w[h][0] >> 14) & 3u, q[h], st, sb, o);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          *reinterpret_cast<f32x4_t*>(bs + swz_f32(col + j, 2 * seg)) = f32x4_t{o[j][0], o[j][1], o[j][2], o[j][3]};
-          *reinterpret_cast<f32x4_t*>(bs + swz_f32(col + j, 2 * seg + 1)) = f32x4_t{o[j][4], o[j][5], o[j][6], o[j][7]};
-        }
       } else {
         u32x4_t o[4];
         decode_cell<kCF == kCellCols>((w[h][0] >> 14) & 3u, q[h], st, sb, o);
@@ -706,10 +687,8 @@ __device__ __forceinline__ void tile_dequant_block(const mtc_tile_desc& d, void*
       }
     }
   };
-  // 16-byte pieces of the tile's rows: 8 per row in bf16, 16 in fp32
-  constexpr int SH = F32 ? 4 : 3, EPP = F32 ? 4 : 8;   // log2 pieces per row, elements per piece
   auto write_out = [&](int ks) __attribute__((always_inline)) {
-    if constexpr (OUT == kOutRows) {
+    if constexpr (kRows) {
       const int n = ct * kTN + 4 * (t & 63);               // N % 32 == 0: a segment is wholly inside or outside N
       if (n >= d.N) return;
 #pragma unroll
@@ -728,14 +707,12 @@ __device__ __forceinline__ void tile_dequant_block(const mtc_tile_desc& d, void*
       return;
     }
 #pragma unroll
-    for (int i = 0; i < (kTN << SH) / 256; ++i) {
-      const int piece = t + 256 * i, row = piece >> SH, seg = piece & ((1 << SH) - 1);
+    for (int i = 0; i < kTN * 8 / 256; ++i) {
+      const int piece = t + 256 * i, row = piece >> 3, seg = piece & 7;   // 16-byte pieces, 8 per row
       const int n = ct * kTN + row;
-      if (n < d.N) {
-        const int64_t e = (int64_t)n * ldw + (int64_t)ks * kTK + seg * EPP;
-        const u32x4_t v = *reinterpret_cast<const u32x4_t*>(bs + (F32 ? swz_f32(row, seg) : swz(row, seg)));
-        *reinterpret_cast<u32x4_t*>(reinterpret_cast<unsigned char*>(Wt) + e * (F32 ? 4 : 2)) = v;
-      }
+      if (n < d.N)
+        *reinterpret_cast<u32x4_t*>(reinterpret_cast<__bf16*>(Wt) + (int64_t)n * ldw + (int64_t)ks * kTK + seg * 8) =
+            *reinterpret_cast<const u32x4_t*>(bs + swz(row, seg));
     }
   };
   // step i: descriptors wa, payload qa; step i + 1: descriptors wb, payload qb
@@ -762,18 +739,12 @@ __device__ __forceinline__ void tile_dequant_block(const mtc_tile_desc& d, void*
 template <int kCF>
 __global__ __launch_bounds__(256) void k_tile_dequant_bf16(const mtc_tile_desc d, __bf16* __restrict__ Wt,
                                                           int64_t ldw, int spb) {
-  tile_dequant_block<kCF, kOutWtBf16>(d, Wt, ldw, spb);
-}
-
-template <int kCF>
-__global__ __launch_bounds__(256) void k_tile_dequant_f32(const mtc_tile_desc d, float* __restrict__ Wt,
-                                                         int64_t ldw, int spb) {
-  tile_dequant_block<kCF, kOutWtF32>(d, Wt, ldw, spb);
+  tile_dequant_block<kCF, false>(d, Wt, ldw, spb);
 }
 
 template <int kCF>
 __global__ __launch_bounds__(256) void k_tile_dequant_rows(const mtc_tile_desc d, float* __restrict__ W, int spb) {
-  tile_dequant_block<kCF, kOutRows>(d, W, d.N, spb);
+  tile_dequant_block<kCF, true>(d, W, d.N, spb);
 }
 
 // Up to kMaxGroup matrices that read the same X, in one launch of each kernel: member i owns
@@ -1232,9 +1203,7 @@ constexpr int kDecodeOnceMinRows = 512;
 constexpr int64_t kDecodeOnceMinMacs = (int64_t)1 << 28;   // below: one launch more costs more than it saves
 // The GEMM runs without a workspace: the algorithms hipBLASLt picks first for the bf16 shapes timed
 // here need none when allowed 32 MiB (and run as fast), and one without a workspace can neither
-// leave a memset node in a captured graph nor split K with atomic sums. (Some fp32 shapes' first
-// algorithms need one, 896 x 4864 x 1024: 4 MB; with none allowed those calls find no algorithm and
-// keep the tile kernel.)
+// leave a memset node in a captured graph nor split K with atomic sums.
 constexpr size_t kBlasWsBytes = 0;
 std::atomic<int> g_decode_once{1};
 
@@ -1302,7 +1271,7 @@ struct Plan {
 
 std::mutex g_mu;
 std::map<int, hipblasLtHandle_t> g_handles;                                   // per device
-std::map<std::tuple<int, int, int, int, int, int64_t, int64_t, int64_t, bool>, Plan> g_plans;
+std::map<std::tuple<int, int, int, int, int, int64_t, int64_t, int64_t>, Plan> g_plans;
 
 // Whether work enqueued on st is being captured into a graph.
 bool capturing(hipStream_t st) {
@@ -1312,11 +1281,10 @@ bool capturing(hipStream_t st) {
 
 // The GEMM plan of a shape on the current device, made once (the heuristic's first algorithm
 // among those needing at most kBlasWsBytes of workspace, so a shape always runs the same
-// algorithm); nullptr when the library or an algorithm is missing. f32: fp32 operands (the
-// exact W_hat and fp32 X) instead of bf16 ones. setup: whether the library may be opened and
+// algorithm); nullptr when the library or an algorithm is missing. setup: whether the library may be opened and
 // the device's handle made here, which allocates; a caller whose stream is being captured passes
 // false and gets nullptr (the tile kernel runs) until a call outside a capture has made them.
-const Plan* plan_for(int M, int N, int K, int64_t ldw, int64_t ldb, int64_t ldy, int ydt, bool f32, bool setup) {
+const Plan* plan_for(int M, int N, int K, int64_t ldw, int64_t ldb, int64_t ldy, int ydt, bool setup) {
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) return nullptr;
   if (!setup) {
@@ -1327,7 +1295,7 @@ const Plan* plan_for(int M, int N, int K, int64_t ldw, int64_t ldb, int64_t ldy,
   const Api& L = api();
   if (!L.ok) return nullptr;
   std::lock_guard<std::mutex> lock(g_mu);
-  const auto key = std::make_tuple(dev, M, N, K, ydt, ldw, ldb, ldy, f32);
+  const auto key = std::make_tuple(dev, M, N, K, ydt, ldw, ldb, ldy);
   auto it = g_plans.find(key);
   if (it != g_plans.end()) return it->second.ok ? &it->second : nullptr;
   Plan& p = g_plans[key];
@@ -1344,8 +1312,8 @@ const Plan* plan_for(int M, int N, int K, int64_t ldw, int64_t ldb, int64_t ldy,
   if (L.desc_create(&p.op, HIPBLAS_COMPUTE_32F, HIP_R_32F) != HIPBLAS_STATUS_SUCCESS ||
       L.desc_set(p.op, HIPBLASLT_MATMUL_DESC_TRANSA, &ta, sizeof(ta)) != HIPBLAS_STATUS_SUCCESS ||
       L.desc_set(p.op, HIPBLASLT_MATMUL_DESC_TRANSB, &tb, sizeof(tb)) != HIPBLAS_STATUS_SUCCESS ||
-      L.layout_create(&p.a, f32 ? HIP_R_32F : HIP_R_16BF, (uint64_t)K, (uint64_t)N, ldw) != HIPBLAS_STATUS_SUCCESS ||
-      L.layout_create(&p.b, f32 ? HIP_R_32F : HIP_R_16BF, (uint64_t)K, (uint64_t)M, ldb) != HIPBLAS_STATUS_SUCCESS ||
+      L.layout_create(&p.a, HIP_R_16BF, (uint64_t)K, (uint64_t)N, ldw) != HIPBLAS_STATUS_SUCCESS ||
+      L.layout_create(&p.b, HIP_R_16BF, (uint64_t)K, (uint64_t)M, ldb) != HIPBLAS_STATUS_SUCCESS ||
       L.layout_create(&p.c, yt, (uint64_t)N, (uint64_t)M, ldy) != HIPBLAS_STATUS_SUCCESS)
     return nullptr;
   hipblasLtMatmulPreference_t pref = nullptr;
@@ -1377,8 +1345,7 @@ int gemm(const Plan* p, const void* Wt, const void* Xb, void* Y, void* ws, hipSt
 const lt::Plan* decode_once_plan(const mtc_tile_desc* d, int x_dtype, int64_t ldx, int64_t ldy, int y_dtype, int M,
                                  bool setup) {
   if (!decode_once_shape(d, M) || !g_decode_once.load(std::memory_order_relaxed)) return nullptr;
-  return lt::plan_for(M, d->N, d->K, decode_once_ldw(d), needs_staging(d, x_dtype) ? d->K : ldx, ldy, y_dtype, false,
-                      setup);
+  return lt::plan_for(M, d->N, d->K, decode_once_ldw(d), needs_staging(d, x_dtype) ? d->K : ldx, ldy, y_dtype, setup);
 }
 
 // Stage X (if needed), decode W_hat into Wt, run the GEMM; ws holds decode_once_bytes.
@@ -1413,26 +1380,6 @@ int decode_once_call(const mtc_tile_desc* d, const void* X, int x_dtype, int64_t
   const int rc = check_launch("k_tile_dequant_bf16");
   if (rc) return rc;
   return lt::gemm(p, Wt, xb, Y, w, st);
-}
-
-// ---- decode once for fp32 results (mtc_gemm_f32): the exact W_hat in fp32, then hipBLASLt's
-// fp32 GEMM (fp32 products and sums), for calls with at least kDecodeOnceF32MinRows rows,
-// kDecodeOnceF32MinMacs multiply-adds, no output column permutation and K of at most kDecodeOnceF32MaxK.
-// The tile kernel is the faster one at every size (4096 x 4096 QT @ 4.5, M = 256, 1024, 2048: 53, 165, 284 us
-// against 85, 248, 476; 1024 x 4096, M = 1024: 49 against 76); the path stays where K <= 1024 for callers
-// that read the decoded W_hat from the workspace, as the decode-once tests do.
-constexpr int kDecodeOnceF32MinRows = 256;
-constexpr int kDecodeOnceF32MaxK = 1024;
-constexpr int64_t kDecodeOnceF32MinMacs = (int64_t)1 << 32;
-
-bool decode_once_f32_shape(const mtc_tile_desc* d, int M) {
-  return !d->col_perm && d->K <= kDecodeOnceF32MaxK && M >= kDecodeOnceF32MinRows &&
-         (int64_t)M * d->K * d->N >= kDecodeOnceF32MinMacs;
-}
-
-// Workspace of the fp32 path: Wt (N x ldw fp32), then X gathered through row_perm (M x K fp32).
-size_t decode_once_f32_bytes(const mtc_tile_desc* d, int M) {
-  return round256((size_t)d->N * decode_once_ldw(d) * 4) + (d->row_perm ? round256((size_t)M * d->K * 4) : 0);
 }
 
 // Workspace of a group: per member, its staged X (if any) then its split-K partials, each on a
@@ -1806,7 +1753,7 @@ int launch_gemm_batch(const void* host_plan, const void* device_plan, hipStream_
     // the plan's choice stands (made when it was built; the switch may have changed since)
     const GemmBatchItem& e = hitems[once_list[j]];
     const lt::Plan* p = lt::plan_for(h->M, e.d.N, e.d.K, decode_once_ldw(&e.d),
-                                     needs_staging(&e.d, h->x_dtype) ? e.d.K : e.ldx_src, e.ldy, h->y_dtype, false,
+                                     needs_staging(&e.d, h->x_dtype) ? e.d.K : e.ldx_src, e.ldy, h->y_dtype,
                                      !lt::capturing(st));
     if (!p) return fail(MTC_E_LAUNCH, "batch item %u: no GEMM plan for its decode-once path", once_list[j]);
     rc = decode_once_call(&e.d, e.Xsrc, h->x_dtype, e.ldx_src, e.Y, h->M,
@@ -1878,9 +1825,8 @@ F32Plan f32_plan(const mtc_tile_desc* d, int M, int max_tm = 128, int max_splits
 size_t f32_stage_bytes(const mtc_tile_desc* d, int M) {
   return d->row_perm ? ((size_t)M * d->K * 4 + 255) / 256 * 256 : 0;
 }
-size_t f32_ws_bytes(const mtc_tile_desc* d, int M) {
-  const F32Plan p = f32_plan(d, M);
-  return f32_stage_bytes(d, M) + (p.splits > 1 ? (size_t)p.splits * M * d->N * 4 : 0);
+size_t f32_partial_bytes(const mtc_tile_desc* d, int M, const F32Plan& p) {
+  return p.splits > 1 ? (size_t)p.splits * M * d->N * 4 : 0;
 }
 
 namespace {
@@ -1914,8 +1860,7 @@ int launch_f32(const mtc_tile_desc* d, const F32Plan& p, const float* X, int64_t
 
 MTC_API size_t mtc_gemm_f32_workspace_bytes(const mtc_tile_desc* d, int M) {
   if (check_tile_desc(d) || M <= 0) return 0;
-  const size_t tiles = f32_ws_bytes(d, M);
-  return decode_once_f32_shape(d, M) ? std::max(tiles, decode_once_f32_bytes(d, M)) : tiles;
+  return f32_stage_bytes(d, M) + f32_partial_bytes(d, M, f32_plan(d, M));
 }
 
 MTC_API int mtc_tile_plan(const mtc_tile_desc* d, int M, int fp32_results, int* tile_rows, int* k_splits) {
@@ -1947,11 +1892,8 @@ MTC_API int mtc_gemm_f32(const mtc_tile_desc* d, const float* X, int64_t ldx, fl
   if (ldx >= (int64_t)1 << 25)
     return fail(MTC_E_SHAPE, "ldx=%lld too large for 32-bit X tile offsets", (long long)ldx);
   hipStream_t st = reinterpret_cast<hipStream_t>(hip_stream);
-  const lt::Plan* once = nullptr;
-  if (decode_once_f32_shape(d, M) && g_decode_once.load(std::memory_order_relaxed))
-    once = lt::plan_for(M, d->N, d->K, decode_once_ldw(d), d->row_perm ? d->K : ldx, ldy, MTC_DTYPE_F32, true,
-                        !lt::capturing(st));
-  const size_t stage = f32_stage_bytes(d, M), need = once ? decode_once_f32_bytes(d, M) : f32_ws_bytes(d, M);
+  F32Plan p = f32_plan(d, M);
+  const size_t stage = f32_stage_bytes(d, M), need = stage + f32_partial_bytes(d, M, p);
   if (need && (!workspace || workspace_bytes < need))
     return fail(MTC_E_WORKSPACE, "fp32 tile workspace of %zu bytes needed, %zu given", need,
                 workspace ? workspace_bytes : 0);
@@ -1959,37 +1901,6 @@ MTC_API int mtc_gemm_f32(const mtc_tile_desc* d, const float* X, int64_t ldx, fl
     return fail(MTC_E_WORKSPACE, "workspace not 256-byte aligned");
   const float* xa = X;
   int64_t lda = ldx;
-  if (once) {
-    // the exact W_hat in fp32, X gathered through row_perm after it, then the fp32 GEMM
-    float* const Wt = reinterpret_cast<float*>(workspace);
-    const int64_t ldw = decode_once_ldw(d);
-    if (d->row_perm) {
-      float* xp = reinterpret_cast<float*>(reinterpret_cast<char*>(workspace) + round256((size_t)d->N * ldw * 4));
-      hipLaunchKernelGGL(k_stage_x_f32, dim3((unsigned)((d->K / 4 + kStageThreads - 1) / kStageThreads), (unsigned)M),
-                         dim3(kStageThreads), 0, st, X, ldx, d->row_perm, xp, d->K);
-      rc = check_launch("k_stage_x_f32");
-      if (rc) return rc;
-      xa = xp;
-      lda = d->K;
-    }
-    // K-steps per block: two blocks per CU by LDS (a 64 KB fp32 tile)
-    const int64_t n_steps = (int64_t)d->n_col_tiles * d->n_ksteps;
-    const int spb = (int)std::min<int64_t>(8, std::max<int64_t>(1, n_steps / (2 * kFillCUs)));
-    const dim3 grid((unsigned)d->n_col_tiles, (unsigned)((d->n_ksteps + spb - 1) / spb));
-    switch (cell_format(d)) {
-      case kCellFp32:
-        hipLaunchKernelGGL(k_tile_dequant_f32<kCellFp32>, grid, dim3(256), 0, st, *d, Wt, ldw, spb);
-        break;
-      case kCellCols:
-        hipLaunchKernelGGL(k_tile_dequant_f32<kCellCols>, grid, dim3(256), 0, st, *d, Wt, ldw, spb);
-        break;
-      default:
-        hipLaunchKernelGGL(k_tile_dequant_f32<kCellBf16>, grid, dim3(256), 0, st, *d, Wt, ldw, spb);
-    }
-    rc = check_launch("k_tile_dequant_f32");
-    if (rc) return rc;
-    return lt::gemm(once, Wt, xa, Y, nullptr, st);
-  }
   if (stage) {
     float* xp = reinterpret_cast<float*>(workspace);
     hipLaunchKernelGGL(k_stage_x_f32, dim3((unsigned)((d->K / 4 + kStageThreads - 1) / kStageThreads), (unsigned)M),
@@ -1999,7 +1910,6 @@ MTC_API int mtc_gemm_f32(const mtc_tile_desc* d, const float* X, int64_t ldx, fl
     xa = xp;
     lda = d->K;
   }
-  F32Plan p = f32_plan(d, M);
   if (lda >= ((int64_t)1 << 30) / p.tm)      // a block's X rows span 4 GiB: a lower tile, in the workspace of this plan
     p = f32_plan(d, M, lda >= (int64_t)1 << 24 ? 32 : 64, p.splits);
   float* part = p.splits > 1 ? reinterpret_cast<float*>(reinterpret_cast<char*>(workspace) + stage) : nullptr;
