@@ -1041,14 +1041,18 @@ bool needs_staging(const mtc_tile_desc* d, int x_dtype) { return d->row_perm || 
 
 constexpr int kFillCUs = 256;             // blocks that fill the chip (one tile block per CU)
 constexpr int kMinStepsPerSplit = 2;
-constexpr double kReduceBytesPerUs = 5.0e6;   // split-K partials written + read, bytes per microsecond
 constexpr double kReduceLaunchUs = 3.0;   // the reduction pass's own launch
 
 // Time of one K-step of a tile block by its row-tile height, and of its launch to the first step's data
 // (kBlockUs). 256 rows (k_gemm_tile) 1.9-2.4 us; the short kernels at 4096 x 4096 in 32, 64 and 128 rows
 // without a K split: 57.8, 67.6 and 85.8 us for 64 steps. The reduction: 4.4 us with 2 splits, 8.4 with
 // 8 (M = 100, 64-row tiles).
+// Calls of more than 256 rows price k_gemm_tile without a launch time and the partials (bytes written + read
+// a microsecond) at 4e6: with 4 us and 5e6 they split sooner, and of 48 calls with another plan for it those
+// that went from 1 split to 2 or 3 lost 3 to 17 % (352 x 3040, M = 339: 18.5 -> 22.1 us; 416 x 1888, M = 466:
+// 24.7 -> 25.9), and none won more than 4 % but those whose old splits did not fit an XCD.
 constexpr double kBlockUs = 4.0;
+constexpr double kReduceBytesPerUs = 5.0e6, kTallReduceBytesPerUs = 4.0e6;
 inline double step_us(int tm) { return tm == 256 ? 2.0 : tm == 128 ? 1.28 : tm == 64 ? 0.97 : 0.85; }
 
 struct TilePlan {
@@ -1063,15 +1067,16 @@ struct TilePlan {
 // blocks past one per CU, and the split-K partial traffic (written by the tile blocks, read by the
 // reduction). Rounds are counted on the fullest XCD: 22 column tiles are 3 on seven XCDs and 1 on the
 // eighth, and 11 splits of them, 242 blocks, are two rounds there (2072 x 5472 uniform, M = 40: 20.9 us
-// with 11 splits, 15.2 with 7 to 8, 15.5 with 6).
+// with 11 splits, 15.2 with 7 to 8, 15.5 with 6; 4192 x 320 QT, M = 283: 32.9 with 33, 22.6 with 22).
 TilePlan tile_plan(const mtc_tile_desc* d, int M) {
   const int64_t full = (int64_t)((M + kTM - 1) / kTM) * d->n_col_tiles;
   if (full >= kFillCUs) return {kTM, 1, d->n_ksteps};
-  const double split_bytes = 2.0 * 4.0 * (double)M * d->N;     // one partial, written and read
+  const bool tall = M > kTM;
+  const double split_us = 2.0 * 4.0 * (double)M * d->N / (tall ? kTallReduceBytesPerUs : kReduceBytesPerUs);   // a partial
   TilePlan best{kTM, 1, d->n_ksteps};
   double best_t = 1e300;
   for (int tm : {256, 128, 64, 32}) {
-    if (tm < kTM && M > kTM) break;                         // shorter tiles timed for M <= 256 only
+    if (tm < kTM && tall) break;                            // shorter tiles timed for M <= 256 only
     if (tm == 32 && M > 32) break;                          // (two 32-row tiles decode every weight twice)
     const int64_t n_tiles = (int64_t)((M + tm - 1) / tm) * d->n_col_tiles;
     int max_s = n_tiles >= kFillCUs ? 1 : (int)((kFillCUs + n_tiles - 1) / n_tiles);
@@ -1080,8 +1085,8 @@ TilePlan tile_plan(const mtc_tile_desc* d, int M) {
       const int per = (d->n_ksteps + s - 1) / s;
       const int s_eff = (d->n_ksteps + per - 1) / per;
       const double rounds = std::ceil((double)((n_tiles + kXcds - 1) / kXcds * s_eff) / (kFillCUs / kXcds));
-      const double t = rounds * (per * step_us(tm) + kBlockUs) +
-                       (s_eff > 1 ? s_eff * split_bytes / kReduceBytesPerUs + kReduceLaunchUs : 0.0);
+      const double t = rounds * (per * step_us(tm) + (tall ? 0.0 : kBlockUs)) +
+                       (s_eff > 1 ? s_eff * split_us + kReduceLaunchUs : 0.0);
       if (t < best_t) {
         best_t = t;
         best = {tm, s_eff, per};

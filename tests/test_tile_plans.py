@@ -42,3 +42,19 @@ def _one_round_of_the_chip_only(M, N, rows, splits):
 def test_f32_plan_counts_rounds_on_the_fullest_xcd(plan):
     for M, K, N in [(545, 1664, 4224), (155, 2464, 2816)] + list(_shapes(3000, 17, 1024, 1)):
         assert not _one_round_of_the_chip_only(M, N, *plan(M, K, N, True)), (M, K, N, plan(M, K, N, True))
+
+
+def test_tall_bf16_plans_keep_their_pricing(plan):
+    """Calls of more than 256 rows: 2 us a K-step, partials at 4 bytes a picosecond and 3 us for their reduction.
+    Shapes that a dearer block splits sooner and slower stay unsplit."""
+    for M, K, N in ((339, 352, 3040), (466, 416, 1888), (409, 416, 2400), (443, 512, 3168), (465, 768, 6048)):
+        assert plan(M, K, N, False) == (256, 1), (M, K, N)
+    for M, K, N in _shapes(2000, 257, 4096, 2):
+        tiles, steps = -(-M // 256) * -(-N // 256), -(-K // 64)
+        best = (1e300, 1)
+        for s in range(1, 1 if tiles >= CUS else 1 + max(1, min(-(-CUS // tiles), steps // 2))):
+            per = -(-steps // s)
+            s = -(-steps // per)
+            rounds = -(-(-(-tiles // XCDS) * s) // (CUS // XCDS))
+            best = min(best, (rounds * per * 2.0 + (s * 8.0 * M * N / 4e6 + 3.0 if s > 1 else 0.0), s))
+        assert plan(M, K, N, False) == (256, best[1]), (M, K, N)
