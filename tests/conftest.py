@@ -114,3 +114,64 @@ def kind_mix_stream(K=4096, N=32, seed=24):
     scales4 = (2.0 ** rng.randint(-8, 0, size=(K // 4, N // 4))).astype(np.float32)
     codes = lambda S, P, ii, jj, sc: rng.randint(-(1 << (P - 1)), 1 << (P - 1), size=(ii.size, S, S))
     return pack_levels((K, N), (4,), {4: leaf4}, {4: modes4}, {4: scales4}, codes, chunk_rows=K, merge_kinds=False)
+
+
+def cell_format_matrices(shapes):
+    """{(name, form): (MTCMatrix, oracle's W_hat)} for every cell format of the tile stream: a quadtree (bf16 scale
+    pairs), a permuted one (gathered columns), one with P16 codes and uniform blocks (fp32 scales)."""
+    from oracle import mtc_oracle as O
+    from tensorpack_amd.core.allocation import rd_allocate
+    from tensorpack_amd.core.permutation import PermutedQuadtreeRD
+    from tensorpack_amd.core.quadtree import QuadtreeRD
+    from tensorpack_amd.kernels.gemm import MTCMatrix
+    out = {}
+    for shape, (K, N) in shapes.items():
+        W = outlier_matrix(K + N, K, N)
+        h = np.exp(np.random.RandomState(K).randn(K))
+        for form, bits in (("qt", 4.0), ("qtp", 3.5), ("p16", 11.0)):
+            a = (PermutedQuadtreeRD if form == "qtp" else QuadtreeRD)(W, h, (32, 16, 8, 4)).select(bits)
+            i = getattr(a, "inner", a)
+            if form == "qtp":
+                W_hat = O.permuted_qt_dequant(W, a.row_perm, a.col_perm, i.sizes, i.leaf, i.modes, i.scales)
+            else:
+                W_hat = O.qt_dequant(W, i.sizes, i.leaf, i.modes, i.scales)
+            out[shape, form] = MTCMatrix.from_quadtree(a, W), W_hat
+        al = rd_allocate(W, 4.5, None, 32)
+        out[shape, "uniform"] = (MTCMatrix.from_allocation(W, al.modes, al.scales, 32),
+                                 O.uniform_to_array(W, al.modes, al.scales, 32))
+    return out
+
+
+def leaf_matrix(form, K, N, seed):
+    """(MTCMatrix, W_hat) of 32 x 32 leaves, each of a random code width (P0 and P16 among them), without an
+    allocation's search: form qt, qtp (rows and columns permuted) or uniform (fp32 scales)."""
+    from tensorpack_amd.core.permutation import PermutedQTAllocation
+    from tensorpack_amd.core.quadtree import QTAllocation
+    from tensorpack_amd.kernels.gemm import MTCMatrix
+    rng = np.random.RandomState(seed)
+    g = (K // 32, N // 32)
+    P = rng.choice([0, 2, 3, 4, 5, 6, 8, 16], size=g)
+    top = np.where(P > 0, 2 ** np.maximum(P - 1, 0), 0)
+    scales = ((2.0 ** -P) * rng.uniform(1.0, 2.0, g)).astype(np.float32)
+    if form != "uniform":
+        scales = (scales.view(np.uint32) & 0xFFFF0000).view(np.float32)
+    up = lambda a: np.repeat(np.repeat(a, 32, axis=0), 32, axis=1)
+    q = rng.randint(-(1 << 15), 1 << 15, size=(K, N)) % np.maximum(2 * up(top), 1) - up(top)
+    W = (q * up(scales)).astype(np.float32)
+    if form == "uniform":
+        return MTCMatrix.from_allocation(W, P.astype(np.uint8), scales, 32), W
+    a = QTAllocation((32,), {32: np.ones(g, bool)}, {32: P}, {32: scales}, None, int((P * 1024).sum()), weights=W)
+    if form == "qt":
+        return MTCMatrix.from_quadtree(a), W
+    pr, pc = rng.permutation(K), rng.permutation(N)
+    back = np.empty_like(W)
+    back[np.ix_(pr, pc)] = W
+    return MTCMatrix.from_quadtree(PermutedQTAllocation(a, pr, pc, a.total_bits)), back
+
+
+def tile_rows(tiles, M, fp32):
+    """Rows per output tile that the tile kernels choose for M rows of X (mtc_tile_plan)."""
+    import ctypes
+    rows, splits = ctypes.c_int32(), ctypes.c_int32()
+    assert tiles.lib.mtc_tile_plan(ctypes.byref(tiles.desc), M, int(fp32), ctypes.byref(rows), ctypes.byref(splits)) == 0
+    return rows.value

@@ -5,12 +5,10 @@ import numpy as np
 import pytest
 
 from oracle import mtc_oracle as O
-from tensorpack_amd.core.allocation import rd_allocate
-from tensorpack_amd.core.permutation import PermutedQuadtreeRD
-from tensorpack_amd.core.quadtree import QTAllocation, QuadtreeRD
+from tensorpack_amd.core.quadtree import QTAllocation
 from tensorpack_amd.kernels.gemm import MTCMatrix
 
-from conftest import outlier_matrix
+from conftest import cell_format_matrices, leaf_matrix, tile_rows
 
 pytestmark = pytest.mark.gpu
 
@@ -20,22 +18,7 @@ SHAPES = {"ragged": (992, 288), "deep": (4096, 544)}
 
 @pytest.fixture(scope="module")
 def mats():
-    out = {}
-    for shape, (K, N) in SHAPES.items():
-        W = outlier_matrix(K + N, K, N)
-        h = np.exp(np.random.RandomState(K).randn(K))
-        for form, bits in (("qt", 4.0), ("qtp", 3.5), ("p16", 11.0)):
-            a = (PermutedQuadtreeRD if form == "qtp" else QuadtreeRD)(W, h, (32, 16, 8, 4)).select(bits)
-            i = getattr(a, "inner", a)
-            if form == "qtp":
-                W_hat = O.permuted_qt_dequant(W, a.row_perm, a.col_perm, i.sizes, i.leaf, i.modes, i.scales)
-            else:
-                W_hat = O.qt_dequant(W, i.sizes, i.leaf, i.modes, i.scales)
-            out[shape, form] = MTCMatrix.from_quadtree(a, W), W_hat
-        al = rd_allocate(W, 4.5, None, 32)
-        out[shape, "uniform"] = (MTCMatrix.from_allocation(W, al.modes, al.scales, 32),
-                                 O.uniform_to_array(W, al.modes, al.scales, 32))
-    return out
+    return cell_format_matrices(SHAPES)
 
 
 def _tol(K):
@@ -51,24 +34,29 @@ def test_f32_tiles_at_every_height(gpu, mats, shape, form):
     m, W_hat = mats[shape, form]
     K = W_hat.shape[0]
     t = m.device_tiles(gpu)
-    for M in (1, 17, 31, 32, 33, 64, 65, 100, 128, 129, 250):
+    heights = set()
+    for M in (1, 17, 31, 32, 33, 64, 65, 100, 128, 129, 250) + ((700, 703, 2999, 3000, 3009) if shape == "ragged" else ()):
         print("f32 split", shape, form, M, flush=True)
+        heights.add(tile_rows(t, M, True))
         X = (np.random.RandomState(M).randn(M, K) * np.exp(3 * np.random.RandomState(K).randn(K))).astype(np.float32)
         Y = t.gemm_f32(torch.from_numpy(X).to(gpu)).cpu().numpy()
         err = O.relative_frobenius_error(O.qt_gemm_f64(X, W_hat), Y)
         assert err <= _tol(K), (M, err)
+    assert heights == ({32, 64, 128} if shape == "ragged" else {32, 64})
 
 
 @pytest.mark.parametrize("form", ["qt", "qtp", "uniform"])
-@pytest.mark.parametrize("M", [20, 64, 100])
-def test_f32_tiles_infinities_nan_and_range(gpu, mats, form, M):
+@pytest.mark.parametrize("M,rows", [(20, 32), (64, 32), (100, 32), (700, 64), (3000, 128)])
+def test_f32_tiles_infinities_nan_and_range(gpu, mats, form, M, rows):
     """Infinities and NaN go where the fp64 product has them, the other rows keep their values; finite
-    values near the end of fp32's range (bf16's rounding would make them infinite) give finite results,
-    and subnormal ones are not worse than an absolute 2^-126 a product."""
+    values near the end of fp32's range (the scaled planes would be infinite) give finite results, and
+    subnormal ones lose nothing but the rounding of subnormal sums. Blocks of every height, whose plain
+    fp32 pass takes 1 to 8 turns."""
     import torch
     m, W_hat = mats["ragged", form]
     K = W_hat.shape[0]
     t = m.device_tiles(gpu)
+    assert tile_rows(t, M, True) == rows
     X = np.random.RandomState(M).randn(M, K).astype(np.float32)
     Z = X.copy()
     Z[3, 5], Z[7, 100], Z[M - 1, K - 1] = np.inf, np.nan, -np.inf
@@ -78,11 +66,11 @@ def test_f32_tiles_infinities_nan_and_range(gpu, mats, form, M):
         ref = Z.astype(np.float64) @ W_hat.astype(np.float64)
     assert np.array_equal(np.isnan(Y), np.isnan(ref)) and np.array_equal(np.isinf(Y), np.isinf(ref))
     assert np.array_equal(np.sign(Y[np.isinf(Y)]), np.sign(ref[np.isinf(ref)]))
-    rows = np.setdiff1d(np.arange(M), [3, 7, M - 1])
-    assert O.relative_frobenius_error(ref[rows], Y[rows]) <= np.sqrt(K) * 2.0 ** -25    # an fma chain of K steps
+    rest = np.setdiff1d(np.arange(M), [3, 7, M - 1])
+    assert O.relative_frobenius_error(ref[rest], Y[rest]) <= np.sqrt(K) * 2.0 ** -25    # an fma chain of K steps
     big = np.zeros((M, K), np.float32)
-    big[np.arange(M), np.arange(M)] = np.float32(3.4e38)
-    small = np.abs(W_hat[:M]).max(axis=1, keepdims=True) < 0.99
+    big[np.arange(M), np.arange(M) % K] = np.float32(3.4e38)
+    small = np.abs(W_hat[np.arange(M) % K]).max(axis=1, keepdims=True) < 0.99
     Yb = t.gemm_f32(torch.from_numpy(big).to(gpu)).cpu().numpy()
     with np.errstate(over="ignore"):
         want = (big.astype(np.float64) @ W_hat.astype(np.float64)).astype(np.float32)
@@ -91,7 +79,8 @@ def test_f32_tiles_infinities_nan_and_range(gpu, mats, form, M):
     tiny = (X * 1e-38).astype(np.float32)
     Yt = t.gemm_f32(torch.from_numpy(tiny).to(gpu)).cpu().numpy().astype(np.float64)
     ref = tiny.astype(np.float64) @ W_hat.astype(np.float64)
-    assert np.abs(Yt - ref).max() <= K * 2.0 ** -126 * np.abs(W_hat).max()
+    # the bar of the others on the largest output, and half a subnormal step for each of at most 32 partials and sums
+    assert np.abs(Yt - ref).max() <= np.sqrt(K) * 2.0 ** -25 * np.abs(ref).max() + 32 * 2.0 ** -149
 
 
 def _flat(W, P, scales, S=32):
@@ -181,3 +170,22 @@ def test_f32_small_magnitudes(gpu, mats, form):
         Y = w.gemm_f32(torch.from_numpy(X).to(gpu)).cpu().numpy()
         up = 2.0 ** 112
         assert O.relative_frobenius_error(O.qt_gemm_f64(X, W_hat) * up, Y.astype(np.float64) * up) <= _tol(K)
+
+
+def test_f32_x_rows_far_apart(gpu):
+    """X rows so far apart that 128 or 64 of them span 4 GiB: the call takes a lower tile, in the workspace of its
+    usual plan."""
+    import torch
+    K = N = 4096
+    M = 250
+    t = leaf_matrix("qt", K, N, 3)[0].device_tiles(gpu)
+    assert tile_rows(t, M, True) == 128
+    X = torch.randn(M, K, device=gpu)
+    want = X.double() @ t.dequant().double()
+    for ldx in ((1 << 23) + 4, (1 << 24) + 4):
+        print("f32 far rows", ldx, flush=True)
+        Z = torch.empty(M * ldx, device=gpu).as_strided((M, K), (ldx, 1))
+        Z.copy_(X)
+        Y = t.gemm_f32(Z).double()
+        assert ((Y - want).norm() / want.norm()).item() <= _tol(K), ldx
+        del Z

@@ -5,12 +5,9 @@ import numpy as np
 import pytest
 
 from oracle import mtc_oracle as O
-from tensorpack_amd.core.allocation import rd_allocate
-from tensorpack_amd.core.permutation import PermutedQuadtreeRD
-from tensorpack_amd.core.quadtree import QuadtreeRD
 from tensorpack_amd.kernels.gemm import MTCMatrix, mtc_gemm_group
 
-from conftest import outlier_matrix
+from conftest import cell_format_matrices, leaf_matrix, tile_rows
 
 pytestmark = pytest.mark.gpu
 
@@ -20,22 +17,7 @@ SHAPES = {"ragged": (992, 288), "one": (64, 256), "deep": (4096, 544)}
 
 @pytest.fixture(scope="module")
 def mats():
-    out = {}
-    for shape, (K, N) in SHAPES.items():
-        W = outlier_matrix(K + N, K, N)
-        h = np.exp(np.random.RandomState(K).randn(K))
-        for form, bits in (("qt", 4.0), ("qtp", 3.5), ("p16", 11.0)):
-            a = (PermutedQuadtreeRD if form == "qtp" else QuadtreeRD)(W, h, (32, 16, 8, 4)).select(bits)
-            i = getattr(a, "inner", a)
-            if form == "qtp":
-                W_hat = O.permuted_qt_dequant(W, a.row_perm, a.col_perm, i.sizes, i.leaf, i.modes, i.scales)
-            else:
-                W_hat = O.qt_dequant(W, i.sizes, i.leaf, i.modes, i.scales)
-            out[shape, form] = MTCMatrix.from_quadtree(a, W), W_hat
-        al = rd_allocate(W, 4.5, None, 32)
-        out[shape, "uniform"] = (MTCMatrix.from_allocation(W, al.modes, al.scales, 32),
-                                 O.uniform_to_array(W, al.modes, al.scales, 32))
-    return out
+    return cell_format_matrices(SHAPES)
 
 
 @pytest.mark.parametrize("shape", SHAPES)
@@ -60,3 +42,27 @@ def test_short_tiles_at_every_height(gpu, mats, shape, form, x):
         # a group's members split K as the single call does: the same sums in the same order
         for Z in mtc_gemm_group(Xg, [m, m], compute="bf16"):
             assert torch.equal(Z, Y), M
+
+
+@pytest.mark.parametrize("form", ["qt", "qtp", "uniform"])
+@pytest.mark.parametrize("x", ["fp32", "bf16"])
+def test_128_row_tiles(gpu, form, x):
+    """Sizes that take 128-row tiles, the last of 72 rows, with K split: a single call (X in place, staged or rounded
+    on the way), a group and a batch (which run the height of the single calls)."""
+    import torch
+    from tensorpack_amd.device import GemmBatch
+    K, N, M = 1504, 5472, 200
+    m, W_hat = leaf_matrix(form, K, N, 7)
+    t = m.device_tiles(gpu)
+    assert tile_rows(t, M, False) == 128
+    print("128-row tiles", form, x, flush=True)
+    X = torch.from_numpy(np.random.RandomState(M).randn(M, K).astype(np.float32)).to(gpu)
+    ref = X.bfloat16().double() @ torch.from_numpy(W_hat).to(gpu).bfloat16().double()
+    Xg = X if x == "fp32" else X.bfloat16()
+    Y = t.gemm_bf16(Xg, out_dtype=torch.float32)
+    assert ((Y - ref).norm() / ref.norm()).item() <= np.sqrt(K) * 2.0 ** -24      # as above
+    assert torch.equal(t.gemm_bf16(Xg, out_dtype=torch.bfloat16), Y.bfloat16())
+    for Z in mtc_gemm_group(Xg, [m, m], compute="bf16"):
+        assert torch.equal(Z, Y)
+    for Z in GemmBatch([t, t.clone()], [Xg, Xg]).launch():
+        assert torch.equal(Z, Y)
