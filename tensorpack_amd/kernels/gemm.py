@@ -30,14 +30,13 @@ from ..core.precision import (_BlockErrors, block_codes, block_scale, negotiate_
 from ..core.quadtree import QTAllocation
 from ..core.types import PrecisionMode
 from ..packer import LAYOUT_MX, LAYOUT_V1, PanelStream, check_permutation, pack_levels, weight_codes
-from ..tilestream import TileStream, pack_tiles
+from ..tilestream import TileStream, pack_tiles, tile_stream_fits
 
 DECODE_MAX_M = 16             # M at or below this takes the fp32 decode kernel under compute="auto"
 F32_DECODE_MAX_M = 16         # fp32 compute above this many rows runs the fp32 tile path (mtc_gemm_f32)
 DECODE_X_LDS_BYTES = 64 * 1024   # on-chip budget for the gathered X rows of one vector-path decode block
 DECODE_MFMA_X_LDS_BYTES = 128 * 1024   # the same for a matrix-core decode block (M tiles of 8 or 16 rows)
 DECODE_LDS_BYTES = 160 * 1024    # per-block LDS of gfx950
-TILE_DEQUANT_MAX_WEIGHTS = 1 << 29       # any mix of code widths (2 bytes a weight at most) fits a 2 GiB tile stream
 UNIFORM_BLOCK_SIZES = (4, 8, 16, 32)   # block sizes of the uniform form the device stream holds
 
 
@@ -573,15 +572,16 @@ class MTCMatrix:
     def dequant_device(self, device=None):
         """W_hat as a (K, N) fp32 device tensor in the original channel order. From the tile
         stream (4096 x 4096 QT-P @ 4.25: 17.9 us against 280 us from the panel stream, whose
-        units scatter 4-byte stores through col_perm; it also packs in half the time), unless
-        only a panel stream is on the device already, or the matrix may not fit the tile stream."""
+        units scatter 4-byte stores through col_perm),
+        unless only a panel stream is on the device already (packing tiles would cost this call more
+        than its 0.3 ms), or the matrix may not fit the tile stream."""
         from ..device import DeviceStream, require_gpu
         dev = require_gpu(device)
         if (str(dev), "tiles") not in self._dev:
             for key, held in list(self._dev.items()):
                 if key[0] == str(dev) and isinstance(held, DeviceStream):
                     return held.dequant()
-            if self.shape[0] * self.shape[1] > TILE_DEQUANT_MAX_WEIGHTS:
+            if not tile_stream_fits(self.shape):
                 return self.device_stream(None, dev).dequant()
         return self.device_tiles(dev).dequant()
 

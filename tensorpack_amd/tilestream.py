@@ -97,6 +97,14 @@ def _scale_words(s: np.ndarray, fp32: bool) -> np.ndarray:
     return bits >> 16
 
 
+def tile_stream_fits(shape: Tuple[int, int]) -> bool:
+    """Whether every allocation of a K x N matrix packs within the kernels' 32-bit byte offsets: at most 2 bytes of
+    payload and 1 byte of cells (gathered columns) a weight, of whole K-steps and column tiles."""
+    K, N = shape
+    padded = -(-K // TILE_ROWS) * TILE_ROWS * -(-N // TILE_COLS) * TILE_COLS
+    return 2 * padded + 4 * PAYLOAD_PAD <= 0x7FFFFFFF
+
+
 def pack_tiles(shape: Tuple[int, int], sizes: Sequence[int], leaf: Dict[int, np.ndarray],
                modes: Dict[int, np.ndarray], scales: Dict[int, np.ndarray], codes_of,
                scale_format: str = "bf16", row_perm: Optional[np.ndarray] = None,

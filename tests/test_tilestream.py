@@ -11,7 +11,7 @@ from tensorpack_amd.core.allocation import rd_allocate
 from tensorpack_amd.core.permutation import PermutedQuadtreeRD
 from tensorpack_amd.core.quadtree import QuadtreeRD
 from tensorpack_amd.kernels.gemm import MTCMatrix
-from tensorpack_amd.tilestream import CELLS, CLS_DWORDS, CLS_Z, decode_tiles
+from tensorpack_amd.tilestream import CELLS, CLS_DWORDS, CLS_Z, PAYLOAD_PAD, decode_tiles, tile_stream_fits
 
 from conftest import outlier_matrix
 
@@ -134,3 +134,33 @@ def test_gathered_columns_for_permuted_matrices(K, N, budget):
     with pytest.raises(ValueError):
         pack_tiles(lv.shape, lv.sizes, lv.leaf, lv.modes, lv.scales, lv.codes_of, lv.scale_format, lv.row_perm,
                    None, gather_cols=True)
+
+
+@pytest.mark.parametrize("K,N", [(1 << 23, 32), (1 << 22, 32), (1 << 21, 32), (32, 1 << 25), (32, 1 << 23), (32768, 16384),
+                                 (32768, 32768), (32768, 16128), (8, 32)])
+def test_tile_stream_fits_what_packs(K, N):
+    """The rule admits exactly the shapes whose widest possible stream (all P16) packs: cells and payload of whole
+    K-steps and column tiles, in 31-bit byte offsets (pack_tiles refuses more)."""
+    steps = -(-K // 64) * -(-N // 256)
+    widest = (steps * CELLS * int(CLS_DWORDS.max()) + PAYLOAD_PAD) * 4
+    assert tile_stream_fits((K, N)) == (widest <= 0x7FFFFFFF and steps * CELLS * 4 * 8 <= 0x7FFFFFFF)
+
+
+def test_dequant_device_leaves_the_tile_stream_to_what_fits(monkeypatch):
+    """A matrix too large for the tile stream (here by its padding: 32 columns of a 256-column tile) is rebuilt from
+    the panel stream, as every matrix was before there was a tile dequantizer."""
+    from tensorpack_amd import device
+
+    class Stream:
+        def __init__(self, name):
+            self.name = name
+
+        def dequant(self):
+            return self.name
+    monkeypatch.setattr(device, "require_gpu", lambda d=None: "gpu")
+    monkeypatch.setattr(MTCMatrix, "device_tiles", lambda self, dev=None: Stream("tiles"))
+    monkeypatch.setattr(MTCMatrix, "device_stream", lambda self, *a, **k: Stream("panels"))
+    for shape, want in (((1 << 23, 32), "panels"), ((4096, 4096), "tiles"), ((32768, 32768), "panels")):
+        m = MTCMatrix.__new__(MTCMatrix)
+        m.shape, m._dev = shape, {}
+        assert m.dequant_device() == want, shape
