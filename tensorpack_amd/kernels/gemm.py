@@ -572,7 +572,7 @@ class MTCMatrix:
     def dequant_device(self, device=None):
         """W_hat as a (K, N) fp32 device tensor in the original channel order. From the tile
         stream (4096 x 4096 QT-P @ 4.25: 17.9 us against 280 us from the panel stream, whose
-        units scatter 4-byte stores through col_perm),
+        units scatter 4-byte stores through col_perm; packing it the first time takes no longer),
         unless only a panel stream is on the device already (packing tiles would cost this call more
         than its 0.3 ms), or the matrix may not fit the tile stream."""
         from ..device import DeviceStream, require_gpu
