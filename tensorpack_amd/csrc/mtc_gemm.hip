@@ -206,60 +206,6 @@ __device__ __forceinline__ void decode_cell(uint32_t cls, const u32x4_t* pw, con
   }
 }
 
-// decode_cell in fp32: out[j][r] = (u - offset) * s for column j, row r (the exact W_hat value,
-// fma(u, s, -offset * s), before any bf16 rounding).
-template <bool PC>
-__device__ __forceinline__ void decode_cell_f32(uint32_t cls, const u32x4_t* pw, const float (&st)[4],
-                                                const float (&sb)[4], float (&out)[4][8]) {
-  constexpr int NS = PC ? 4 : 1;
-  float ct[NS], cb[NS];
-  auto offset_terms = [&](float off) __attribute__((always_inline)) {
-#pragma unroll
-    for (int j = 0; j < NS; ++j) {
-      ct[j] = -off * st[j];
-      cb[j] = -off * sb[j];
-    }
-  };
-  // rows 0-3 from the bytes of `top`, rows 4-7 from `bot`
-  auto bytes = [&](int j, uint32_t top, uint32_t bot, int k) __attribute__((always_inline)) {
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      out[j][r] = __builtin_fmaf((float)((top >> (8 * r)) & 0xFFu), st[k], ct[k]);
-      out[j][4 + r] = __builtin_fmaf((float)((bot >> (8 * r)) & 0xFFu), sb[k], cb[k]);
-    }
-  };
-  if (cls == 0) {
-    offset_terms(8.0f);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const uint32_t x = pw[0][j];
-      bytes(j, opaque(x & 0x0F0F0F0Fu), opaque((x >> 4) & 0x0F0F0F0Fu), PC ? j : 0);
-    }
-  } else if (cls == 1) {
-    offset_terms(128.0f);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) bytes(j, pw[j >> 1][(2 * j) & 3], pw[j >> 1][(2 * j + 1) & 3], PC ? j : 0);
-  } else if (cls == 2) {
-    offset_terms(32768.0f);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int k = PC ? j : 0;
-      const uint32_t v[4] = {pw[j].x, pw[j].y, pw[j].z, pw[j].w};
-#pragma unroll
-      for (int h = 0; h < 4; ++h) {
-        const float s = h < 2 ? st[k] : sb[k], c = h < 2 ? ct[k] : cb[k];
-        out[j][2 * h] = __builtin_fmaf((float)(v[h] & 0xFFFFu), s, c);
-        out[j][2 * h + 1] = __builtin_fmaf((float)(v[h] >> 16), s, c);
-      }
-    }
-  } else {
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-#pragma unroll
-      for (int r = 0; r < 8; ++r) out[j][r] = 0.0f;
-  }
-}
-
 // Output tile (rt, ct) of a launch of one matrix from its block index bx: each XCD (bx % 8)
 // takes a contiguous range of tile ids. Without an output column permutation the ids run
 // over groups of kRowGroup row tiles, row tile fastest, so the blocks in flight on one XCD
@@ -667,8 +613,11 @@ __device__ __forceinline__ void tile_dequant_block(const mtc_tile_desc& d, void*
         // code times scale, as the panel stream's dequantizer computes it (one rounded product: exact for
         // bf16 scales; no negative zeros in a quadtree W_hat, whose levels are summed into +0.0)
         const float one[4] = {1.0f, 1.0f, 1.0f, 1.0f};
+        uint32_t pw[16];
+#pragma unroll
+        for (int e = 0; e < 16; ++e) pw[e] = q[h][e >> 2][e & 3];
         float o[4][8];
-        decode_cell_f32<kCF == kCellCols>((w[h][0] >> 14) & 3u, q[h], one, one, o);
+        decode_cols_f32<false, 4>((w[h][0] >> 14) & 3u, pw, one, one, o);
 #pragma unroll
         for (int r = 0; r < 8; ++r) {
           f32x4_t v;

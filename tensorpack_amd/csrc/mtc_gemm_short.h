@@ -78,7 +78,8 @@ __device__ __forceinline__ void split_planes(const float* v, u32x4_t& hi, u32x4_
   }
 }
 
-// decode_cell_f32 for NC columns: pw holds their 4 NC dwords (a class W4 cell's first NC, a W8 cell's first 2 NC).
+// decode_cell in fp32 for NC columns: out[j][r] = fma(u, s, -offset * s) for column j, row r, the exact W_hat value before
+// any bf16 rounding. pw holds their 4 NC dwords (a class W4 cell's first NC, a W8 cell's first 2 NC).
 template <bool PC, int NC>
 __device__ __forceinline__ void decode_cols_f32(uint32_t cls, const uint32_t (&pw)[4 * NC], const float (&st)[NC],
                                                 const float (&sb)[NC], float (&out)[NC][8]) {
