@@ -287,7 +287,7 @@ int mtc_tile_dequant(const mtc_tile_desc* d, float* W_out, void* hip_stream);
 /* Bytes of prefill workspace for M rows of X of dtype x_dtype (256-byte aligned
  * workspace; contents need no initialisation): M*K*2 (rounded up to 256) when X may
  * be staged as bf16 first (fp32 X, or a row permutation to gather; fp32 X without a
- * permutation, with 16-byte aligned rows, in the 64- and 128-row tiles of short X is
+ * permutation, with 16-byte aligned rows, in the tiles of at most 128 rows of short X is
  * rounded to bf16 by the tile kernel itself and leaves that area unused), plus
  * splits*M*N*4 when the output has too few 256 x 256 tiles to fill the chip and the
  * K steps are split over blocks (fp32 partial tiles, summed in a fixed order).

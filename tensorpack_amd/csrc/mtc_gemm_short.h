@@ -4,13 +4,14 @@
 //
 // Block = one TM x 256 output tile over a run of K-steps. Every wave decodes and every
 // wave multiplies: a thread takes one cell of a step (512 cells; half a cell where a block has 1024
-// threads), whose descriptor was loaded four steps and whose payload three steps ahead, decodes it into
-// the B tile in LDS, and after the barrier the waves run the step's MFMAs. With few rows a step's MFMAs take less time than its
-// decode and its memory latency; four waves that decode for eight that multiply (k_gemm_tile) then leave
-// most of a CU's issue slots idle. Sums run in k_gemm_tile's order: the same bits for the same K splits.
-// Measured against k_gemm_tile's blocks of 64 or 128 rows, with the plan of tile_plan, us a call: 2072 x 5472
-// uniform, M = 40: 23.0 -> 14.9; 6144 x 1024 QT, M = 160: 27.7 -> 18.9; 4096 x 4096 QT-P, M = 128: 29.0 -> 25.6;
-// M = 256 of 4096 x 4096 QT 29.1 -> 29.0 (bound by the 8 splits' partials and their reduction, about 14 us).
+// threads), whose descriptor was loaded four steps and whose payload three steps ahead (two and one for
+// fp32 results in 128 rows), decodes it into the B tile in LDS, and after the barrier the waves run the
+// step's MFMAs. With few rows a step's MFMAs take less time than its decode and its memory latency; four
+// waves that decode for eight that multiply (k_gemm_tile) then leave most of a CU's issue slots idle. Sums run in k_gemm_tile's order: the same bits for the same K splits.
+// Measured against k_gemm_tile's blocks of 64 or 128 rows and their plan, us a call replayed from a graph of ten:
+// 2072 x 5472 uniform, M = 40: 23.0 -> 14.9 (20.9 with the old plan's 11 splits; eager, bound by the host, 23.6 ->
+// 21.2); 6144 x 1024 QT, M = 160: 27.7 -> 18.9; 4096 x 4096 QT-P, M = 128: 29.0 -> 25.6; 4096 x 4096 QT, M = 256:
+// 29.1 -> 29.0 (64 rows, 4 splits: 24.4 us of 16 steps, first data and partials, 5.0 of reduction).
 //
 // fp32 results on the bf16 matrix cores. A float is cut into bf16 planes by truncation, hi + mid + lo,
 // each the upper half of what the planes before left (8 + 8 + 8 significant bits: exact, mid below 2^-7 and
@@ -28,6 +29,10 @@
 // Error against fp64, 2-norm, 4096 x 4096 QT @ 4.5 (an fma chain in K order: the fp32 MFMAs of 16-row tiles):
 // M = 100 1.2e-7 (6.0e-7), M = 2048 3.4e-7 (1.0e-6); X and W positive, M = 2048 3.0e-7 (8.6e-7), 8192 x 4096
 // 4.3e-7 (1.2e-6); X times 2^-124 1.2e-7 (6.1e-7); one product alone 2.5e-8 (2.5e-8).
+// Time, from a graph, against the 16-row tiles: 4096 x 4096 QT-P @ 4.25, M = 100, 120.8 -> 42.7 us; QT, M = 1024
+// 565 -> 171, M = 2048 1128 -> 307 (224 TFLOP/s of fp32 results; the library's fp32 product 248 and 475 us). A K-step takes 1.9,
+// 2.9 or 5.0 us at 32, 64 or 128 rows: decode and LDS stores, then the MFMAs (1.3 us at 64 rows), one after
+// the other, as two buffers of three planes do not fit the LDS; the matrix pipes are busy 0.26 at M = 100.
 #pragma once
 
 enum { kXBf16, kXRound, kXSplit };   // X: bf16 / fp32 rounded to bf16 / fp32 cut into three planes
@@ -39,7 +44,7 @@ template <int XM, int TM>
 struct ShortTile {
   static_assert(TM == 128 || TM == 64 || TM == 32, "row tiles of 128, 64 or 32 rows");
   static constexpr bool split = XM == kXSplit;
-  // split: 1024 threads decode a step faster than 512; 128 rows need 128 registers a thread for their sums alone
+  // split: 1024 threads, but at 128 rows, where the two accumulators would leave them 64 registers for all else
   static constexpr int threads = split && TM < 128 ? 1024 : 512, waves = threads / 64;
   static constexpr int ct = kCells * 4 / threads;            // columns of a cell that one thread decodes
   static constexpr int planes = split ? 3 : 1;

@@ -352,8 +352,8 @@ class DeviceTiles:
         return out
 
     def gemm_f32(self, X, out=None):
-        """Y = X @ W_hat in fp32 on the matrix core (mtc_gemm_f32): the exact W_hat, fp32
-        products and sums, for M from a few rows up."""
+        """Y = X @ W_hat in fp32 on the matrix core (mtc_gemm_f32): the exact W_hat and X
+        in bf16 planes, whose products are exact, with fp32 sums, for M from a few rows up."""
         torch = _torch()
         _need(X.dim() == 2 and X.stride(1) == 1 and X.dtype == torch.float32 and X.shape[1] == self.K
               and X.device == self.device, f"X must be (M, {self.K}) fp32 row-major on {self.device}")

@@ -617,7 +617,7 @@ def _kernel_layout(X):
 
 def _gemm_f32(B: "MTCMatrix", Xf, dev):
     """fp32 Y = Xf @ W_hat: the decode kernels over the panel stream up to F32_DECODE_MAX_M rows,
-    the fp32 matrix-core tile path above (4096 x 4096 QT-P, M = 16: 24 us on either; M = 64: 33 against 73)."""
+    the fp32 tile path above (4096 x 4096 QT-P, M = 16: 23 us on either; M = 32: 25 against 40, M = 64: 31 against 76)."""
     M = Xf.shape[0]
     if M > F32_DECODE_MAX_M:
         if Xf.stride(0) % 4 or Xf.data_ptr() % 16:   # the tile kernel reads rows in 16-byte pieces

@@ -357,8 +357,8 @@ def test_gemm_bf16(gpu, allocs, name, M, xdtype):
 @pytest.mark.parametrize("name", [c[0] for c in CASES])
 @pytest.mark.parametrize("M", [1, 5, 16, 17, 40])
 def test_gemm_f32_tiles(gpu, allocs, name, M):
-    """The fp32 matrix-core path over the tile stream (mtc_gemm_f32: exact W_hat, fp32 products
-    and sums, 16-row tiles, split K): Y within the fp32 bar, every call the same bits, and X = I
+    """The fp32 matrix-core path over the tile stream (mtc_gemm_f32: exact W_hat and X in bf16
+    planes, fp32 sums, 32-row tiles at these sizes, split K): Y within the fp32 bar, every call the same bits, and X = I
     returns W_hat itself (one product per output, exact in fp32)."""
     import torch
     W, a, m = allocs[name]
