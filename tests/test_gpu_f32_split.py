@@ -189,3 +189,21 @@ def test_f32_x_rows_far_apart(gpu):
         Y = t.gemm_f32(Z).double()
         assert ((Y - want).norm() / want.norm()).item() <= _tol(K), ldx
         del Z
+
+
+@pytest.mark.parametrize("form", ["qt", "qtp", "p16", "uniform"])
+def test_f32_large_sums(gpu, mats, form):
+    """Finite sums past 2^80, which overflow the scaled accumulators: those tiles come from the plain pass."""
+    import torch
+    m, W_hat = mats["ragged", form]
+    K = W_hat.shape[0]
+    t = m.device_tiles(gpu)
+    for M in (20, 700, 3000):
+        X = np.random.RandomState(M).randn(M, K).astype(np.float32)
+        X[: M // 2] *= np.float32(2.0 ** 90)
+        print("f32 large sums", form, M, flush=True)
+        Y = t.gemm_f32(torch.from_numpy(X).to(gpu)).cpu().numpy()
+        ref = X.astype(np.float64) @ W_hat.astype(np.float64)
+        assert np.isfinite(Y).all()
+        for rows in (slice(0, M // 2), slice(M // 2, M)):
+            assert O.relative_frobenius_error(ref[rows], Y[rows]) <= np.sqrt(K) * 2.0 ** -25    # an fma chain of K steps
