@@ -22,8 +22,8 @@ def mats():
 
 
 def _tol(K):
-    # each output: 6 MFMA sums per 16 rows of K, each rounded once to fp32 (a random walk of half-ulp
-    # steps on the running sum), and the plane products left out, below 2^-24 of their product
+    # each output: sums of 16 rows of K, rounded once to fp32 (a random walk of half-ulp steps on the running sum);
+    # held to six of them, as if every plane pair went to the one accumulator
     return (np.sqrt(6 * K / 16) + 2) * 2.0 ** -25
 
 
