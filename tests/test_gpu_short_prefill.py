@@ -5,7 +5,7 @@ import numpy as np
 import pytest
 
 from oracle import mtc_oracle as O
-from tensorpack_amd.kernels.gemm import MTCMatrix, mtc_gemm_group
+from tensorpack_amd.kernels.gemm import mtc_gemm_group
 
 from conftest import cell_format_matrices, leaf_matrix, tile_rows
 
